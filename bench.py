@@ -38,7 +38,7 @@ VALU_PEAK_TOPS = 39.3    # 256 CU x 64 lanes x 2.4 GHz int32 lane-ops/s
 MFMA_FP4_PEAK_TOPS = 10100.0  # MI355X dense FP4 matrix ops/s (10.1 PFLOP/s)
 NW_OPS_PER_CELL = 13     # nominal int ops per in-band DP cell
 KMER_KERNELS = ("kmer_profile", "kmer_tile", "kmer_cand_pop", "kmer_cand_sort", "kmer_cand", "kmer_sort")
-NW_KERNELS = ("nw_bucket", "nw_band_reg", "nw_band_sliced", "nw_generic", "nw_filter")
+NW_KERNELS = ("nw_bucket", "nw_band_pk", "nw_band_reg", "nw_band_sliced", "nw_generic", "nw_filter")
 # the NW launches of one step run concurrently on side streams; this event
 # pair on the main stream brackets all of them (fork to join)
 NW_PHASE = "nw_dp_phase"
@@ -462,7 +462,7 @@ def main():
     # filter): 2 ops x kdim per pair
     kdim = r["tile_bits"]
     kmer_tile_tops = kt["units"] * 2 * kdim / (kt["total_ms"] * 1e-3) / 1e12 if kt["total_ms"] else 0
-    dp_launches = sum(kern[k]["launches"] for k in ("nw_band_reg", "nw_band_sliced", "nw_generic"))
+    dp_launches = sum(kern[k]["launches"] for k in ("nw_band_pk", "nw_band_reg", "nw_band_sliced", "nw_generic"))
     if phase_ms >= kt["total_ms"] / steps:
         # One DP phase per step: the fused register / sliced family launches run
         # concurrently on the worker streams; the phase is timed fork to join.

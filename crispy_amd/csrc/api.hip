@@ -22,9 +22,13 @@ int set_err(crispy_ctx *ctx, int code, const char *fmt, ...) {
 int ensure(crispy_ctx *ctx, DevBuf &b, size_t bytes) {
   if (bytes == 0) bytes = 256;
   if (b.bytes >= bytes) return CRISPY_OK;
-  if (ctx->mem_limit > 0 && ctx->dev_bytes - (int64_t)b.bytes + (int64_t)bytes > ctx->mem_limit)
+  // the direction scratch has a limit of its own in a served job
+  const bool apart = ctx->scratch_limit >= 0, scratch = &b == &ctx->nw.dirs;
+  const int64_t held = ctx->dev_bytes - (apart && !scratch ? (int64_t)ctx->nw.dirs.bytes : 0);
+  if (apart && scratch ? (int64_t)bytes > ctx->scratch_limit
+                       : ctx->mem_limit > 0 && held - (int64_t)b.bytes + (int64_t)bytes > ctx->mem_limit)
     return set_err(ctx, CRISPY_ERR_NOMEM, "growing a buffer to %zu bytes would take the context past its "
-                   "device memory limit (%lld of %lld bytes held)", bytes, (long long)ctx->dev_bytes,
+                   "device memory limit (%lld of %lld bytes held)", bytes, (long long)held,
                    (long long)ctx->mem_limit);
   if (b.p) {
     CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -132,12 +136,14 @@ static void drain_timers(crispy_ctx *ctx) {
 }
 
 // One block per read: 2-bit codes (A0 G1 T2 C3, other bytes 0 as in
-// kmerMain.cpp:137-152), 16 bases per word, and the all-ACGT flag.
+// kmerMain.cpp:137-152), 16 bases per word, and the all-ACGT flag; the other
+// bytes met are flagged in `other` (256 bits).
 __global__ __launch_bounds__(256) void pack_reads_kernel(const uint8_t *__restrict__ bases,
                                                          const int64_t *__restrict__ off,
                                                          const int64_t *__restrict__ poff,
                                                          uint32_t *__restrict__ pack,
-                                                         uint8_t *__restrict__ clean) {
+                                                         uint8_t *__restrict__ clean,
+                                                         uint32_t *__restrict__ other) {
   const int r = blockIdx.x;
   const int64_t b0 = off[r];
   const int L = (int)(off[r + 1] - b0);
@@ -153,7 +159,10 @@ __global__ __launch_bounds__(256) void pack_reads_kernel(const uint8_t *__restri
       if (p < L) {
         const uint8_t c = bases[b0 + p];
         const uint32_t code = c == 'G' ? 1u : c == 'T' ? 2u : c == 'C' ? 3u : 0u;
-        bad |= !(c == 'A' || c == 'C' || c == 'G' || c == 'T');
+        if (!(c == 'A' || c == 'C' || c == 'G' || c == 'T')) {
+          bad = 1;
+          atomicOr(&other[c >> 5], 1u << (c & 31));
+        }
         word |= code << (2 * t);
       }
     }
@@ -161,6 +170,39 @@ __global__ __launch_bounds__(256) void pack_reads_kernel(const uint8_t *__restri
   }
   bad = __syncthreads_or(bad);
   if (threadIdx.x == 0) clean[r] = bad ? 0 : 1;
+}
+
+// The NW codes of a read set with other bytes: code[c] of each byte, low two
+// bits to `pack`, upper two to `pack_hi` (zero for a read of ACGT only).
+struct ByteCodes {
+  uint8_t code[256];
+};
+__global__ __launch_bounds__(256) void pack_ext_kernel(const uint8_t *__restrict__ bases,
+                                                       const int64_t *__restrict__ off,
+                                                       const int64_t *__restrict__ poff,
+                                                       const uint8_t *__restrict__ clean, const ByteCodes codes,
+                                                       uint32_t *__restrict__ pack, uint32_t *__restrict__ pack_hi) {
+  const int r = blockIdx.x;
+  const int64_t b0 = off[r];
+  const int L = (int)(off[r + 1] - b0);
+  const int64_t w0 = poff[r];
+  const int nw = (int)(poff[r + 1] - w0);
+  const bool plain = clean[r] != 0;
+  for (int w = threadIdx.x; w < nw; w += blockDim.x) {
+    uint32_t lo = 0, hi = 0;
+    if (!plain) {
+      for (int t = 0; t < 16; ++t) {
+        const int p = w * 16 + t;
+        if (p < L) {
+          const uint32_t c = codes.code[bases[b0 + p]];
+          lo |= (c & 3u) << (2 * t);
+          hi |= (c >> 2) << (2 * t);
+        }
+      }
+      pack[w0 + w] = lo;
+    }
+    pack_hi[w0 + w] = hi;
+  }
 }
 
 __global__ void selftest_div_kernel(int maxv, float *out_kmer, float *out_nw) {
@@ -201,7 +243,7 @@ int crispy_ctx_create(int device, crispy_ctx **out) {
             hipEventCreateWithFlags(&ctx->fork_ev, hipEventDisableTiming) == hipSuccess &&
             hipEventCreateWithFlags(&ctx->stage_ev, hipEventDisableTiming) == hipSuccess &&
             hipDeviceGetAttribute(&ctx->cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
-            hipHostMalloc(&ctx->h_hist, 64, hipHostMallocDefault) == hipSuccess;
+            hipHostMalloc(&ctx->h_hist, 256, hipHostMallocDefault) == hipSuccess;
   for (int w = 0; ok && w < kNumWorkers; ++w)
     ok = hipStreamCreate(&ctx->workers[w]) == hipSuccess &&
          hipEventCreateWithFlags(&ctx->join_ev[w], hipEventDisableTiming) == hipSuccess;
@@ -223,7 +265,7 @@ static void release_all(crispy_ctx *ctx) {
                     &ctx->nw.in_pairs, &ctx->nw.keys,      &ctx->nw.keys_alt,  &ctx->nw.idx,
                     &ctx->nw.order,    &ctx->nw.dist,      &ctx->nw.hist,      &ctx->nw.cells,
                     &ctx->nw.flags,    &ctx->nw.sel,       &ctx->nw.nsel,      &ctx->nw.out_pairs,
-                    &ctx->nw.out_dists, &ctx->nw.scratch,  &ctx->nw.plan,      &ctx->nw.stat,
+                    &ctx->nw.out_dists, &ctx->nw.scratch,  &ctx->nw.plan,      &ctx->nw.stat,      &ctx->nw.dirs,
                     &ctx->temp,
                     &ctx->pre.bases,   &ctx->pre.off,      &ctx->pre.freq,     &ctx->pre.keys,
                     &ctx->pre.keys_alt, &ctx->pre.flags,   &ctx->pre.sel,      &ctx->pre.nsel,
@@ -234,7 +276,7 @@ static void release_all(crispy_ctx *ctx) {
                     &ctx->nw.sort_b0,   &ctx->nw.sort_b1,   &ctx->nw.sort_pairs, &ctx->nw.sort_dists};
   for (DevBuf *b : bufs) release(ctx, *b);
   for (auto &r : ctx->reads) {
-    DevBuf *rb[] = {&r.bases, &r.off, &r.len, &r.pack, &r.poff, &r.clean};
+    DevBuf *rb[] = {&r.bases, &r.off, &r.len, &r.pack, &r.poff, &r.clean, &r.pack_hi, &r.other};
     for (DevBuf *b : rb) release(ctx, *b);
   }
 }
@@ -308,6 +350,14 @@ int crispy_ctx_set_mem_limit(crispy_ctx *ctx, int64_t bytes) {
   return CRISPY_OK;
 }
 
+int crispy_ctx_set_scratch_limit(crispy_ctx *ctx, int64_t bytes) {
+  if (!ctx || bytes < -1) return CRISPY_ERR_ARG;
+  ctx->scratch_limit = bytes;
+  return CRISPY_OK;
+}
+
+int64_t crispy_ctx_scratch_bytes(const crispy_ctx *ctx) { return ctx ? (int64_t)ctx->nw.dirs.bytes : 0; }
+
 int64_t crispy_band_cells(int32_t len1, int32_t len2, int32_t band) {
   if (len1 <= 0 || len2 <= 0) return 0;
   if (band <= 1) return (int64_t)len1 * len2;
@@ -347,7 +397,10 @@ int crispy_reads_upload(crispy_ctx *ctx, int slot, const char *bases, const int6
   CRISPY_TRY(ensure(ctx, rs.poff, sizeof(int64_t) * (n + 1)));
   CRISPY_TRY(ensure(ctx, rs.pack, sizeof(uint32_t) * (nwords + 4)));
   CRISPY_TRY(ensure(ctx, rs.clean, (size_t)n + 1));
+  CRISPY_TRY(ensure(ctx, rs.other, 256 / 8));
+  rs.ext = false;
   if (n > 0) {
+    uint32_t other[8] = {};
     CRISPY_HIP(ctx, hipMemcpyAsync(rs.bases.p, bases, rs.nbases, hipMemcpyHostToDevice, ctx->stream));
     CRISPY_HIP(ctx, hipMemcpyAsync(rs.off.p, offsets, sizeof(int64_t) * (n + 1),
                                    hipMemcpyHostToDevice, ctx->stream));
@@ -355,13 +408,33 @@ int crispy_reads_upload(crispy_ctx *ctx, int slot, const char *bases, const int6
                                    hipMemcpyHostToDevice, ctx->stream));
     CRISPY_HIP(ctx, hipMemcpyAsync(rs.poff.p, poff.data(), sizeof(int64_t) * (n + 1),
                                    hipMemcpyHostToDevice, ctx->stream));
+    CRISPY_HIP(ctx, hipMemsetAsync(rs.other.p, 0, sizeof other, ctx->stream));
     pack_reads_kernel<<<n, 256, 0, ctx->stream>>>(rs.bases.as<uint8_t>(), rs.off.as<int64_t>(),
                                                   rs.poff.as<int64_t>(), rs.pack.as<uint32_t>(),
-                                                  rs.clean.as<uint8_t>());
+                                                  rs.clean.as<uint8_t>(), rs.other.as<uint32_t>());
     CRISPY_LAUNCHED(ctx);
     rs.h_clean.assign(n, 0);
     CRISPY_HIP(ctx, hipMemcpyAsync(rs.h_clean.data(), rs.clean.p, n, hipMemcpyDeviceToHost, ctx->stream));
+    CRISPY_HIP(ctx, hipMemcpyAsync(other, rs.other.p, sizeof other, hipMemcpyDeviceToHost, ctx->stream));
     CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    ByteCodes codes = {};
+    codes.code['G'] = 1;
+    codes.code['T'] = 2;
+    codes.code['C'] = 3;
+    int distinct = 0;
+    for (int c = 0; c < 256; ++c)
+      if ((other[c >> 5] >> (c & 31)) & 1u) {
+        if (distinct < 12) codes.code[c] = (uint8_t)(4 + distinct);
+        ++distinct;
+      }
+    rs.ext = slot == CRISPY_READS_NW && distinct > 0 && distinct <= 12;
+    if (rs.ext) {
+      CRISPY_TRY(ensure(ctx, rs.pack_hi, sizeof(uint32_t) * (nwords + 4)));
+      pack_ext_kernel<<<n, 256, 0, ctx->stream>>>(rs.bases.as<uint8_t>(), rs.off.as<int64_t>(), rs.poff.as<int64_t>(),
+                                                  rs.clean.as<uint8_t>(), codes, rs.pack.as<uint32_t>(),
+                                                  rs.pack_hi.as<uint32_t>());
+      CRISPY_LAUNCHED(ctx);
+    }
   }
   rs.all_clean = 1;
   for (int32_t r = 0; r < n; ++r) rs.all_clean &= rs.h_clean[r];

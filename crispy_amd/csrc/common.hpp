@@ -99,6 +99,11 @@ struct ReadStore {
   int32_t minlen = 0;
   int all_clean = 1;
   DevBuf bases, off, len, pack, poff, clean;
+  // NW slot, reads with other bytes than ACGT: the distinct ones get the codes
+  // 4..15 (low two bits in `pack`, upper two in `pack_hi`, same layout); ext
+  // when there are at most 12 of them
+  DevBuf pack_hi, other;
+  bool ext = false;
   std::vector<int32_t> h_len;
   std::vector<uint8_t> h_clean;
   int generation = 0;  // bumped on every upload (invalidates cached profiles)
@@ -147,10 +152,20 @@ struct NwState {
   DevBuf out_pairs, out_dists, scratch;
   DevBuf plan;  // NwPlan of the DP phase (bucket table, family task lists, counters)
   DevBuf stat;  // cells per family (generic last) summed over timed runs
+  DevBuf dirs;  // direction slots of the packed families
   DevBuf csr_rows, csr_cols;  // CSR view of the (i, j)-ordered result
   DevBuf sort_k0, sort_k1, sort_b0, sort_b1, sort_pairs, sort_dists;  // (dist, i, j) sorts
   int slice_width = 0;  // sliced-kernel cells per lane: 0 = cost model, 24 or 32 = forced
-  GraphSegment g_dp, g_filter;  // captured DP phase and filter
+  // Captured DP phases, one per set of kernels (the kernel families that a
+  // job's read lengths and pair count put to work), and the filter.  A job of
+  // another set takes another graph: an instantiated graph is only ever
+  // updated with new arguments of the same kernels, and a server's slots,
+  // whose jobs alternate between a few sets, do not destroy and instantiate
+  // graphs job after job.
+  static constexpr int kDpGraphs = 8;
+  GraphSegment g_dp[kDpGraphs], g_filter;
+  uint64_t dp_kernels[kDpGraphs] = {};
+  int dp_next = 0;  // the entry that a ninth set replaces
   int64_t count = 0;
   int64_t in_count = 0;  // input pairs of the last run (the filter's scan covers them)
   bool valid = false;
@@ -206,6 +221,8 @@ struct crispy_ctx {
   std::map<std::string, KStat> stats;
   int64_t dev_bytes = 0;
   int64_t mem_limit = 0;  // device bytes the buffers may grow to (0: no limit)
+  // bytes that the direction scratch (nw.dirs) may take beside mem_limit (-1: it counts within mem_limit)
+  int64_t scratch_limit = -1;
 };
 
 namespace crispy {

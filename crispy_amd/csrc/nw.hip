@@ -28,6 +28,11 @@
 //   nw_band_sliced: kKbRegMax < kB <= kKbSliceMax, G lanes per pair.
 //   The register and sliced bodies run as wave tasks of a few fused launches
 //   (one per occupancy family), not one launch per kB bucket.
+//   nw_band_pk (nw_pk.hpp): two positions per register in 16-bit keys, the
+//     directions in a scratch of the context.  Takes every kB whose keys fit
+//     16 bits, full alignments (kB = the longer read) and reads with up to 12
+//     distinct other bytes; what is past that, and a call without room for
+//     the scratch, runs in the kernels above and below.
 //   nw_generic_kernel  one lane per pair, the row state in a lane-
 //     interleaved global scratch, raw byte compares.  Any kB, full mode and
 //     reads with other bytes (N, lowercase, ...).
@@ -75,14 +80,15 @@ static BucketKey bucket_key(int kb_lo, int kb_top, int maxlen) {
 // ---------------------------------------------------------------- bucketing
 // Sort key per pair: kB << 11 | R, R = min(L1, L2) the DP's last row with an
 // in-band cell, clamped to 2047, for the register and sliced kernels; all ones
-// for the generic kernel.  The keys are radix-sorted with the pair indices as
+// for the generic kernel (kB past kKbSliceMax; reads with other bytes where
+// the packed kernels do not take them: kB past ext_top).  The keys are radix-sorted with the pair indices as
 // values; the sort is stable, so equal keys keep the (i, j) order of the
 // input and a wave's pairs mostly share read i (one L1).  Per-bucket pair and
 // cell counts are reduced in LDS first (a handful of buckets would serialise
 // global atomics).
 __global__ __launch_bounds__(256) void nw_bucket_kernel(
     const int2 *__restrict__ pairs, int64_t np, const int32_t *__restrict__ len,
-    const uint8_t *__restrict__ clean, int band, BucketKey bk, uint32_t *__restrict__ keys,
+    const uint8_t *__restrict__ clean, int band, int ext_top, BucketKey bk, uint32_t *__restrict__ keys,
     uint32_t *__restrict__ idx, unsigned int *__restrict__ hist,
     unsigned long long *__restrict__ cells) {
   const uint32_t generic_key = (1u << bk.bits) - 1;
@@ -100,19 +106,16 @@ __global__ __launch_bounds__(256) void nw_bucket_kernel(
     uint32_t key = generic_key;
     int bucket = kGenericBucket;
     int64_t nc;
-    if (band >= 2) {
-      const int kb = (L1 + L2) / (2 * band);
-      nc = band_cells(L1, L2, kb);
-      if (kb <= kKbSliceMax && clean[pr.x] && clean[pr.y]) {
-        // rows past the column read's length + kB hold no in-band cell, and
-        // the DP runs its rows over the shorter read (nw_dp.hpp), so it ends
-        // at row min(L1, L2)
-        const int rows = min(L1, L2);
-        key = ((uint32_t)(kb - bk.kb_lo) << bk.rbits) | (uint32_t)min(rows, 2047);
-        bucket = kb;
-      }
-    } else {
-      nc = (int64_t)L1 * L2;
+    // a full alignment is a band that holds every cell: |i - j| <= the longer read
+    const int kb = band >= 2 ? (L1 + L2) / (2 * band) : max(L1, L2);
+    nc = band >= 2 ? band_cells(L1, L2, kb) : (int64_t)L1 * L2;
+    if (kb <= kKbSliceMax && (kb <= ext_top || (clean[pr.x] && clean[pr.y]))) {
+      // rows past the column read's length + kB hold no in-band cell, and
+      // the DP runs its rows over the shorter read (nw_dp.hpp, nw_pk.hpp), so
+      // it ends at row min(L1, L2)
+      const int rows = min(L1, L2);
+      key = ((uint32_t)(kb - bk.kb_lo) << bk.rbits) | (uint32_t)min(rows, 2047);
+      bucket = kb;
     }
     keys[p] = key;
     idx[p] = (uint32_t)p;
@@ -287,10 +290,13 @@ static inline int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::mi
 
 
 using FamilyLaunch = void (*)(hipStream_t, unsigned, const NwFusedArgs &);
-static const FamilyLaunch kFamilyLaunch[kNumFamilies] = {
+static const FamilyLaunch kFamilyLaunch[kFirstPkFamily] = {
     launch_nw_reg_family0, launch_nw_reg_family1, launch_nw_reg_family2, launch_nw_reg_family3,
     launch_nw_sliced_family24, launch_nw_sliced_family32};
-static_assert(kNumFamilies == 6 && kSliceWidths[0] == 24 && kSliceWidths[1] == 32, "one launcher per family");
+static_assert(kFirstPkFamily == 6 && kSliceWidths[0] == 24 && kSliceWidths[1] == 32, "one launcher per family");
+using PkLaunch = void (*)(hipStream_t, unsigned, const NwFusedArgs &, const PkLaunchArgs &);
+static const PkLaunch kPkLaunch[kNumPkFamilies] = {launch_nw_pk_family0, launch_nw_pk_family1, launch_nw_pk_family2,
+                                                   launch_nw_pk_family3};
 
 // ------------------------------------------------------------ DP phase plan
 // One block of 1024 threads, thread b for bucket b: the plan of the DP phase
@@ -300,7 +306,7 @@ static_assert(kNumFamilies == 6 && kSliceWidths[0] == 24 && kSliceWidths[1] == 3
 // last) are added to it for the timers.
 __global__ __launch_bounds__(1024) void nw_plan_kernel(const unsigned int *__restrict__ hist,
                                                        const unsigned long long *__restrict__ cells,
-                                                       int forced, NwPlan *__restrict__ plan,
+                                                       const NwMap map, NwPlan *__restrict__ plan,
                                                        unsigned long long *__restrict__ stat) {
   static_assert(kNumBuckets <= 1024, "one thread per bucket");
   __shared__ uint32_t s_wsum[16];
@@ -334,8 +340,8 @@ __global__ __launch_bounds__(1024) void nw_plan_kernel(const unsigned int *__res
   if (b < kNumBuckets) {
     plan->btab[b] = make_uint2(start, h);
     if (b < kGenericBucket && h) {
-      f = nw_family_of(b, forced);
-      const uint32_t per = (uint32_t)nw_pairs_per_wave(b, f);
+      f = nw_family_of(b, map);
+      const uint32_t per = (uint32_t)nw_pairs_per_wave(b, f, map.pk_cap);
       waves = (h + per - 1) / per;
       mean = (double)cells[b] / (double)h;
       s_live[atomicAdd(&s_nlive, 1)] = b;
@@ -364,52 +370,169 @@ __global__ __launch_bounds__(1024) void nw_plan_kernel(const unsigned int *__res
   if (b < kNumFamilies) {
     plan->ntasks[b] = s_ntasks[b];
     plan->nbuckets[b] = s_nbk[b];
+    plan->next[b] = 0;
   }
   if (stat && b <= kNumFamilies) stat[b] += s_cells[b];
 }
 
-// Grid of family f for np pairs whose kB lies in [kb_lo, kb_hi]: an upper
-// bound on the family's tasks, np over the fewest pairs per wave among the
-// family's kB in that range plus one partial wave per bucket, rounded up to
+// An upper bound on a family's tasks for np pairs: np over the fewest pairs
+// per wave among its kB plus one partial wave per bucket, rounded up to
 // m * 2^e with m < 16 (similar pair counts launch alike and share a captured
-// graph; at most 1/8 of the blocks are spare).  0 if no kB of the range
-// belongs to the family.
-static int64_t family_grid(int f, int64_t np, int kb_lo, int kb_hi, int forced) {
-  int64_t per = 0, buckets = 0;
-  for (int kb = std::max(kb_lo, 0); kb <= std::min(kb_hi, kKbSliceMax); ++kb) {
-    if (nw_family_of(kb, forced) != f) continue;
-    const int64_t p = nw_pairs_per_wave(kb, f);
-    per = per ? std::min(per, p) : p;
-    ++buckets;
-  }
-  if (!buckets) return 0;
-  int64_t g = (np + per - 1) / per + buckets;
+// graph; at most 1/8 of the blocks are spare).
+static int64_t task_grid(int64_t np, int64_t per, int64_t buckets) {
+  const int64_t g = (np + per - 1) / per + buckets;
   int e = 0;
   while ((g >> e) >= 16) ++e;
   return (((g - 1) >> e) + 1) << e;
 }
 
+// Grid of family f for np pairs whose kB lies in [kb_lo, kb_hi]; 0 if no kB of
+// the range belongs to the family.
+static int64_t family_grid(int f, int64_t np, int kb_lo, int kb_hi, const NwMap &map) {
+  int64_t per = 0, buckets = 0;
+  for (int kb = std::max(kb_lo, 0); kb <= std::min(kb_hi, kKbSliceMax); ++kb) {
+    if (nw_family_of(kb, map) != f) continue;
+    const int64_t p = nw_pairs_per_wave(kb, f, map.pk_cap);
+    per = per ? std::min(per, p) : p;
+    ++buckets;
+  }
+  return buckets ? task_grid(np, per, buckets) : 0;
+}
+
+// The packed families' part of one DP phase: which kB they take, and per
+// family the blocks (= direction slots) and their scratch.
+struct PkPlan {
+  NwMap map;
+  unsigned blocks[kNumPkFamilies] = {};
+  PkLaunchArgs args[kNumPkFamilies] = {};
+  int64_t region[kNumWorkers] = {};  // scratch bytes of each worker stream: its families run one after the other
+  int64_t bytes() const {
+    int64_t b = 0;
+    for (int64_t r : region) b += r;
+    return b;
+  }
+};
+// Direction scratch of one context, at most.
+constexpr int64_t kPkScratchBytes = int64_t(4) << 30;
+
+// Worker stream of family f (neighbouring families, which common length
+// spreads put to work together, run side by side).
+static int family_worker(int f) { return f % kNumWorkers; }
+
+// A plan with slices of at most `cap` cells, as many slots as the chip holds
+// waves or `room` bytes hold, and its cost: the longer of one wave's task and
+// the chip's share of all tasks plus most of a last one, in instructions of
+// (rows + 2 lanes) steps of ~35 + 10.5 per cell, for kB evenly spread.
+static double pk_plan_cap(int cus, int64_t np, int band, int maxlen, int kb_lo, int kb_hi, int forced, int64_t room,
+                          int cap, PkPlan &p) {
+  p = PkPlan();
+  p.map = NwMap{forced, -1, cap};
+  // a pair's rows: its shorter read, at most (L1 + L2) / 2 < band (kB + 1)
+  auto rows = [&](int kb) { return (int)std::min<int64_t>(maxlen, band >= 2 ? (int64_t)band * (kb + 1) : kb); };
+  kb_lo = std::max(kb_lo, 0);
+  const int kb_end = std::min(kb_hi, forced ? kKbRegMax : kPkMaxKb);
+  for (int kb = kb_lo; kb <= kb_end && pk_keys_fit(kb, rows(kb), cap); ++kb) p.map.pk_top = kb;
+  if (p.map.pk_top < 0) return 0;
+  double total = 0, longest = 0;
+  int64_t per[kNumPkFamilies] = {}, buckets[kNumPkFamilies] = {};
+  const double pairs = (double)np / (p.map.pk_top - kb_lo + 1);
+  for (int f = 0; f < kNumPkFamilies; ++f) {
+    p.args[f].cap = cap;
+    p.args[f].f16 = true;
+  }
+  for (int kb = kb_lo; kb <= p.map.pk_top; ++kb) {
+    const int lanes = pk_lanes(kb, cap), cells = pk_cells(kb, cap), steps = rows(kb) + 2 * lanes;
+    int f = 0;
+    while (cells > kPkFamilies[f].hi) ++f;
+    PkLaunchArgs &x = p.args[f];
+    per[f] = per[f] ? std::min<int64_t>(per[f], 64 / lanes) : 64 / lanes;
+    ++buckets[f];
+    x.f16 = x.f16 && pk_keys_fit(kb, rows(kb), cap, kPkF16Top);
+    x.words = std::max<int64_t>(x.words, (int64_t)(steps + kPkTraceSteps - 1) / kPkTraceSteps * kPkTraceSteps *
+                                             pk_dir_words(cells) * 64);
+    const double task = steps * (35 + 10.5 * cells);
+    total += pairs / (64 / lanes) * task;
+    longest = std::max(longest, task);
+  }
+  int64_t full = 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    int64_t slots = 0;
+    for (int64_t &r : p.region) r = 0;
+    for (int f = 0; f < kNumPkFamilies; ++f) {
+      if (!p.args[f].words) continue;
+      unsigned &b = p.blocks[f];
+      if (pass == 0)
+        b = (unsigned)std::min(task_grid(np, per[f], buckets[f]), (int64_t)4 * cus * kPkFamilies[f].waves);
+      else
+        b = (unsigned)(b * ((double)room / (double)full));
+      if (!b) return 0;  // no room for a slot of every family
+      int64_t &r = p.region[family_worker(kFirstPkFamily + f)];
+      r = std::max(r, 4 * (int64_t)b * p.args[f].words);
+      slots += b;
+    }
+    full = p.bytes();
+    const double simds = (double)std::min<int64_t>(slots, 4 * cus);
+    const double cost = std::max(longest, total / simds + 0.9 * longest);
+    if (full <= room) return cost;
+    if (room <= 0) return 0;
+  }
+  return 0;
+}
+
+// Slice width: a wider slice has less of the instructions that each step
+// spends beside its cells, a narrower one splits few pairs over more waves and
+// needs less scratch; the cost above picks it.  Over 18 inputs from 123 to 3.3 M
+// pairs the pick was the fastest of the seven widths or within 3 % of it, twice
+// within 15 %; against 16 cells everywhere a step with 3.3 M pairs of 150-550 bp
+// takes 17.3 ms for 19.6, against 40 everywhere 200 pairs of 1 kbp take
+// 0.64 ms for 1.33.
+// Where the scratch is short of a wave per SIMD the unpacked kernels (~1.6x
+// the instructions, no scratch) are the faster ones.
+static PkPlan pk_plan(int cus, int64_t np, int band, int maxlen, int kb_lo, int kb_hi, int forced, int64_t room) {
+  PkPlan none, best;
+  none.map = best.map = NwMap{forced, -1, kPkMaxCells};
+  if (np == 0) return none;
+  room = std::min(room, kPkScratchBytes);
+  double best_cost = 0, free_cost = 0;
+  int top = -1;
+  for (int cap : {kPkMaxCells, 32, 24, 20, 16, 12, 8}) {
+    PkPlan p;
+    const double unbounded = pk_plan_cap(cus, np, band, maxlen, kb_lo, kb_hi, forced, INT64_MAX, cap, p);
+    if (!unbounded || p.map.pk_top < top) break;  // narrower slices reach fewer kB
+    top = p.map.pk_top;
+    if (!free_cost || unbounded < free_cost) free_cost = unbounded;
+    const double cost = p.bytes() <= room ? unbounded
+                                          : pk_plan_cap(cus, np, band, maxlen, kb_lo, kb_hi, forced, room, cap, p);
+    if (cost && (!best_cost || cost < best_cost)) {
+      best_cost = cost;
+      best = p;
+    }
+  }
+  return best_cost && best_cost <= 1.6 * free_cost ? best : none;
+}
+
 // The DP phase's launches after the bucket sort: the plan, then every family
-// that the reads' kB range allows on the worker streams (family f on worker
-// f mod 2: neighbouring families, which common length spreads put to work
-// together, run side by side).  No host read-back and nothing sized by the histogram, so the
+// that the reads' kB range allows on its worker stream.  No host read-back and nothing sized by the histogram, so the
 // sequence can be captured into a graph.  Per-family timers only when not
 // capturing.
 static int enqueue_dp(crispy_ctx *ctx, const NwFusedArgs &args, const unsigned (&grid)[kNumFamilies],
-                      bool capturing) {
+                      const PkPlan &pk, bool capturing) {
   NwState &nw = ctx->nw;
   nw_plan_kernel<<<1, 1024, 0, ctx->stream>>>(nw.hist.as<unsigned int>(), nw.cells.as<unsigned long long>(),
-                                              nw.slice_width, nw.plan.as<NwPlan>(),
+                                              pk.map, nw.plan.as<NwPlan>(),
                                               ctx->timing ? nw.stat.as<unsigned long long>() : nullptr);
   CRISPY_LAUNCHED(ctx);
   CRISPY_TRY(fork_workers(ctx));
   for (int f = 0; f < kNumFamilies; ++f) {
     if (!grid[f]) continue;
-    hipStream_t s = ctx->workers[f % kNumWorkers];
-    const char *name = f >= kNumRegFamilies ? "nw_band_sliced" : "nw_band_reg";
+    hipStream_t s = ctx->workers[family_worker(f)];
+    const char *name = f >= kFirstPkFamily ? "nw_band_pk" : f >= kNumRegFamilies ? "nw_band_sliced" : "nw_band_reg";
     hipEvent_t ev = nullptr;
     if (!capturing) timer_begin(ctx, name, &ev, s);
-    kFamilyLaunch[f](s, grid[f], args);
+    if (f >= kFirstPkFamily)
+      kPkLaunch[f - kFirstPkFamily](s, grid[f], args, pk.args[f - kFirstPkFamily]);
+    else
+      kFamilyLaunch[f](s, grid[f], args);
     CRISPY_LAUNCHED(ctx);
     if (!capturing) timer_end(ctx, name, ev, 0.0, s);
   }
@@ -425,8 +548,9 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   NwState &nw = ctx->nw;
   if (np > 0xFFFFFFFFll) return set_err(ctx, CRISPY_ERR_ARG, "too many pairs in one call");
   // kB = (L1 + L2) / (2 band) of any pair lies in [minlen / band, maxlen / band]
-  const int kb_lo = band >= 2 ? rs.minlen / band : 0;
-  const int kb_hi = band >= 2 ? rs.maxlen / band : -1;
+  // (a full alignment: its longer read)
+  const int kb_lo = band >= 2 ? rs.minlen / band : rs.minlen;
+  const int kb_hi = band >= 2 ? rs.maxlen / band : rs.maxlen;
   CRISPY_TRY(ensure(ctx, nw.keys, sizeof(uint32_t) * (np + 1)));
   CRISPY_TRY(ensure(ctx, nw.keys_alt, sizeof(uint32_t) * (np + 1)));
   CRISPY_TRY(ensure(ctx, nw.idx, sizeof(uint32_t) * (np + 1)));
@@ -444,6 +568,31 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   float *out = nw.dist.as<float>();
   NwPlan *plan = nw.plan.as<NwPlan>();
 
+  // Pairs of reads with other bytes run packed up to ext_top; what the fused
+  // kernels cannot take exists only if the reads allow it.
+  const int64_t generic_bytes = (std::min<int64_t>(np, 32768) + 255) / 256 * 256 * sizeof(int2) * (rs.maxlen + 1);
+  const int64_t later = 24 * (np + 1) + (1 << 20) + (rs.all_clean ? 0 : generic_bytes);  // the filter's buffers
+  const int64_t room = ctx->scratch_limit >= 0 ? ctx->scratch_limit
+                       : ctx->mem_limit > 0    ? ctx->mem_limit - ctx->dev_bytes + (int64_t)nw.dirs.bytes - later
+                                               : kPkScratchBytes;
+  PkPlan pk = pk_plan(ctx->cus, np, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, room);
+  if (pk.bytes() > 0) {
+    const int rc = ensure(ctx, nw.dirs, (size_t)pk.bytes());
+    if (rc == CRISPY_ERR_NOMEM) {  // a device that others fill: the unpacked kernels need no scratch
+      ctx->err.clear();
+      pk = pk_plan(ctx->cus, 0, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, 0);
+    } else if (rc != CRISPY_OK) {
+      return rc;
+    }
+  }
+  for (int f = 0; f < kNumPkFamilies; ++f) {
+    static_assert(kNumWorkers == 2, "the second worker's region follows the first's");
+    pk.args[f].dirs = nw.dirs.as<uint32_t>() + (family_worker(kFirstPkFamily + f) ? pk.region[0] / 4 : 0);
+    pk.args[f].pack_hi = rs.ext ? rs.pack_hi.as<uint32_t>() : nullptr;
+  }
+  const int ext_top = rs.ext ? pk.map.pk_top : -1;
+  const bool maybe_generic = kb_hi > kKbSliceMax || (!rs.all_clean && kb_hi > ext_top);
+
   // bucketing: launched one by one (the radix sort clears its own state
   // with memsets, which stay out of graphs)
   const BucketKey bkey = bucket_key(kb_lo, std::min(kb_hi, kKbSliceMax), rs.maxlen);
@@ -452,7 +601,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   CRISPY_HIP(ctx, hipMemsetAsync(nw.cells.p, 0, sizeof(unsigned long long) * kNumBuckets, ctx->stream));
   timer_begin(ctx, "nw_bucket", &ev);
   nw_bucket_kernel<<<(int)std::min<int64_t>((np + 255) / 256, 1024), 256, 0, ctx->stream>>>(
-      d_pairs, np, rs.len.as<int32_t>(), rs.clean.as<uint8_t>(), band, bkey, nw.keys.as<uint32_t>(),
+      d_pairs, np, rs.len.as<int32_t>(), rs.clean.as<uint8_t>(), band, ext_top, bkey, nw.keys.as<uint32_t>(),
       nw.idx.as<uint32_t>(), nw.hist.as<unsigned int>(), nw.cells.as<unsigned long long>());
   CRISPY_LAUNCHED(ctx);
   size_t tbytes = 0;
@@ -469,7 +618,8 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
                          d_pairs, order, plan, out};
   unsigned grid[kNumFamilies];
   for (int f = 0; f < kNumFamilies; ++f) {
-    const int64_t g = family_grid(f, np, kb_lo, kb_hi, nw.slice_width);
+    const int64_t g = f >= kFirstPkFamily ? pk.blocks[f - kFirstPkFamily]
+                                          : family_grid(f, np, kb_lo, kb_hi, pk.map);
     if (g > 0x7FFFFFFF)
       return set_err(ctx, CRISPY_ERR_ARG, "%lld pairs need %lld wave tasks in one launch; split the call",
                      (long long)np, (long long)g);
@@ -478,16 +628,29 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   std::vector<uintptr_t> key = {
       (uintptr_t)args.pack, (uintptr_t)args.poff, (uintptr_t)args.len, (uintptr_t)args.pairs,
       (uintptr_t)args.order, (uintptr_t)args.plan, (uintptr_t)args.out, (uintptr_t)nw.hist.p,
-      (uintptr_t)nw.cells.p, (uintptr_t)(ctx->timing ? nw.stat.p : nullptr), (uintptr_t)nw.slice_width};
+      (uintptr_t)nw.cells.p, (uintptr_t)(ctx->timing ? nw.stat.p : nullptr), (uintptr_t)nw.slice_width,
+      (uintptr_t)pk.map.pk_top, (uintptr_t)pk.map.pk_cap, (uintptr_t)nw.dirs.p,
+      (uintptr_t)pk.region[0], (uintptr_t)pk.args[0].pack_hi};
   for (unsigned g : grid) key.push_back(g);
+  for (const PkLaunchArgs &k : pk.args) key.push_back((uintptr_t)k.words);
+  uint64_t kernels = rs.ext ? 1 : 2;
+  for (int f = 0; f < kNumFamilies; ++f) kernels |= grid[f] ? uint64_t(4) << f : 0;
+  for (int f = 0; f < kNumPkFamilies; ++f) kernels |= pk.args[f].f16 ? uint64_t(4) << (kNumFamilies + f) : 0;
+  int gi = 0;
+  while (gi < NwState::kDpGraphs && nw.dp_kernels[gi] && nw.dp_kernels[gi] != kernels) ++gi;
+  if (gi == NwState::kDpGraphs) {
+    gi = nw.dp_next;
+    nw.dp_next = (nw.dp_next + 1) % NwState::kDpGraphs;
+    CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));  // its last launch has ended
+    drop_segment(nw.g_dp[gi]);
+  }
+  nw.dp_kernels[gi] = kernels;
   hipEvent_t phase;
   timer_begin(ctx, "nw_dp_phase", &phase);
-  CRISPY_TRY(run_segment(ctx, nw.g_dp, std::move(key), "NW DP phase",
-                         [&](bool capturing) { return enqueue_dp(ctx, args, grid, capturing); }));
-  // Pairs the fused kernels cannot take (full NW, non-ACGT bytes, kB past
-  // kKbSliceMax) exist only if the reads allow them; then their count comes
-  // back from the plan and the generic kernel runs after the families.
-  const bool maybe_generic = band < 2 || !rs.all_clean || rs.maxlen / band > kKbSliceMax;
+  CRISPY_TRY(run_segment(ctx, nw.g_dp[gi], std::move(key), "NW DP phase",
+                         [&](bool capturing) { return enqueue_dp(ctx, args, grid, pk, capturing); }));
+  // Pairs for the generic kernel: their count comes back from the plan, and it
+  // runs after the families.
   if (maybe_generic) {
     uint2 *h_g = reinterpret_cast<uint2 *>(ctx->h_hist);
     CRISPY_HIP(ctx, hipMemcpyAsync(h_g, &plan->btab[kGenericBucket], sizeof(uint2), hipMemcpyDeviceToHost,
@@ -581,7 +744,8 @@ int nw_timer_units(crispy_ctx *ctx, const char *name, double *units) {
   NwState &nw = ctx->nw;
   int lo, hi;  // families [lo, hi); kNumFamilies is the generic kernel
   if (!std::strcmp(name, "nw_band_reg")) lo = 0, hi = kNumRegFamilies;
-  else if (!std::strcmp(name, "nw_band_sliced")) lo = kNumRegFamilies, hi = kNumFamilies;
+  else if (!std::strcmp(name, "nw_band_sliced")) lo = kNumRegFamilies, hi = kFirstPkFamily;
+  else if (!std::strcmp(name, "nw_band_pk")) lo = kFirstPkFamily, hi = kNumFamilies;
   else if (!std::strcmp(name, "nw_generic")) lo = kNumFamilies, hi = kNumFamilies + 1;
   else if (!std::strcmp(name, "nw_dp_phase")) lo = 0, hi = kNumFamilies + 1;
   else return CRISPY_OK;
@@ -695,7 +859,7 @@ static int noalloc_scratch(crispy_ctx *ctx, unsigned char **out) {
 }
 
 void release_graphs(crispy_ctx *ctx) {
-  drop_segment(ctx->nw.g_dp);
+  for (GraphSegment &g : ctx->nw.g_dp) drop_segment(g);
   drop_segment(ctx->nw.g_filter);
   drop_segment(ctx->km.g_profile);
   drop_segment(ctx->km.g_tile);
@@ -942,17 +1106,18 @@ int crispy_nw_dists_noalloc(crispy_ctx *ctx, const int32_t *d_pairs, int64_t npa
   CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
   if (*h_bad) return set_err(ctx, CRISPY_ERR_ARG, "a pair names a read outside [0, %d)", rs.n);
   nw_bucket_kernel<<<(int)std::min<int64_t>((npairs + 255) / 256, 1024), 256, 0, ctx->stream>>>(
-      pairs, npairs, rs.len.as<int32_t>(), rs.clean.as<uint8_t>(), band, bkey, keys, idx, hist, cells);
+      pairs, npairs, rs.len.as<int32_t>(), rs.clean.as<uint8_t>(), band, -1, bkey, keys, idx, hist, cells);
   CRISPY_LAUNCHED(ctx);
   CRISPY_HIP(ctx, rocprim::radix_sort_pairs<RadixOnesweep>(temp, tbytes, keys, keys_alt, idx, order,
                                                            (size_t)npairs, 0, bkey.bits, ctx->stream));
   const NwFusedArgs args{rs.pack.as<uint32_t>(), rs.poff.as<int64_t>(), rs.len.as<int32_t>(),
                          pairs, order, plan, d_dists};
-  nw_plan_kernel<<<1, 1024, 0, ctx->stream>>>(hist, cells, ctx->nw.slice_width, plan, nullptr);
+  const NwMap map{ctx->nw.slice_width, -1, kPkMaxCells};  // the packed families need direction slots
+  nw_plan_kernel<<<1, 1024, 0, ctx->stream>>>(hist, cells, map, plan, nullptr);
   CRISPY_LAUNCHED(ctx);
   CRISPY_TRY(fork_workers(ctx));
-  for (int f = 0; f < kNumFamilies; ++f) {
-    const int64_t g = family_grid(f, npairs, kb_lo, kb_hi, ctx->nw.slice_width);
+  for (int f = 0; f < kFirstPkFamily; ++f) {
+    const int64_t g = family_grid(f, npairs, kb_lo, kb_hi, map);
     if (!g) continue;
     kFamilyLaunch[f](ctx->workers[f % kNumWorkers], (unsigned)g, args);
     CRISPY_LAUNCHED(ctx);

@@ -577,7 +577,7 @@ __device__ __forceinline__ bool nw_task(const NwPlan *__restrict__ plan, const i
   const uint2 e = list[k - 1];
   task.kb = (int)e.x;
   task.bk = plan->btab[e.x];
-  const uint32_t per = (uint32_t)nw_pairs_per_wave(task.kb, f);
+  const uint32_t per = (uint32_t)nw_pairs_per_wave(task.kb, f, 0);
   const uint32_t waves = (task.bk.y + per - 1) / per;
   task.wave = (int)(waves - 1 - (t - e.y));
   return true;

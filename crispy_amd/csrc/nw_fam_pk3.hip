@@ -1,0 +1,11 @@
+// Packed NW family 3: its slice widths (kPkFamilies), one launch for the
+// ACGT-only read sets and one with the upper code bits.
+#include "nw_pk.hpp"
+
+namespace crispy {
+
+void launch_nw_pk_family3(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k) {
+  launch_nw_pk_family<3>(s, blocks, a, k);
+}
+
+}  // namespace crispy

@@ -28,7 +28,45 @@ static_assert(kRegFamilies[0].lo == 0 && kRegFamilies[0].hi + 1 == kRegFamilies[
 // slice_width_for().
 constexpr int kNumSliceWidths = 2;
 constexpr int kSliceWidths[kNumSliceWidths] = {24, 32};
-constexpr int kNumFamilies = kNumRegFamilies + kNumSliceWidths;
+// Packed families (nw_pk.hpp): G = pk_lanes lanes per pair, each two slices of
+// pk_cells positions; one family per range of slice widths.  `cap` bounds the
+// slice width (at most kPkMaxCells): small jobs take narrower slices, so that
+// their few pairs spread over more lanes (pk_plan in nw.hip).
+constexpr int kPkMaxCells = 40;   // 80 state registers: 3 waves per SIMD
+constexpr int kPkMaxLanes = 16;   // lanes per pair
+constexpr int kPkMaxKb = 639;     // 2 kB + 1 positions over kPkMaxLanes x 2 slices of kPkMaxCells
+static_assert(2 * kPkMaxKb + 1 <= 2 * kPkMaxLanes * kPkMaxCells, "the widest band fits the lanes of a pair");
+struct PkFamily {
+  int lo, hi;     // slice widths
+  int waves;      // per SIMD, by registers
+  int ext_waves;  // with the upper code bits
+};
+constexpr int kNumPkFamilies = 4;
+constexpr PkFamily kPkFamilies[kNumPkFamilies] = {{1, 16, 5, 4}, {17, 24, 4, 3}, {25, 32, 4, 3}, {33, kPkMaxCells, 3, 2}};
+constexpr int kFirstPkFamily = kNumRegFamilies + kNumSliceWidths;
+constexpr int kNumFamilies = kFirstPkFamily + kNumPkFamilies;
+constexpr int kPkTraceSteps = 8;  // steps of directions staged in LDS at a time by the trace
+
+__host__ __device__ constexpr int pk_lanes(int kb, int cap) { return (2 * kb + 1 + 2 * cap - 1) / (2 * cap); }
+__host__ __device__ constexpr int pk_cells(int kb, int cap) {
+  return (2 * kb + 1 + 2 * pk_lanes(kb, cap) - 1) / (2 * pk_lanes(kb, cap));
+}
+// 32-bit words of directions per lane and step: 8 cells of both halves each
+__host__ __device__ constexpr int pk_dir_words(int cells) { return (cells + 7) / 8; }
+// The largest key of bucket kb with at most `rows` rows fits 16 bits (nw_pk.hpp:
+// 9 per row from the -4 frame, 7 per position, a margin for the offers).
+__host__ __device__ constexpr bool pk_keys_fit(int kb, int rows, int cap, int key_top = 0xFFFF) {
+  return kb <= kPkMaxKb && pk_lanes(kb, cap) <= kPkMaxLanes &&
+         9 * (rows + 1) + 7 * 2 * pk_lanes(kb, cap) * pk_cells(kb, cap) + 100 <= key_top >> 2;
+}
+constexpr int kPkF16Top = 0x7BFF;  // the largest finite half-precision pattern
+
+// How a DP phase's buckets map to kernels: `forced` slice width of the sliced
+// kernel (0 = cost model), kB up to pk_top run packed with slices of at most
+// pk_cap cells (pk_top -1: none).
+struct NwMap {
+  int forced, pk_top, pk_cap;
+};
 
 __host__ __device__ constexpr int slice_lanes(int kb, int C) { return (2 * kb + 1 + C - 1) / C; }
 
@@ -47,17 +85,22 @@ __host__ __device__ inline int slice_width_for(int kb, int forced) {
   return g24 >= 7 && (27 * 32 + 90) * p24 <= (27 * 24 + 90) * p32 ? 32 : 24;
 }
 
-// Kernel family of bucket kB (kB <= kKbSliceMax) under slice-width policy
-// `forced` (0 = cost model).
-__host__ __device__ inline int nw_family_of(int kb, int forced) {
-  if (kb > kKbRegMax) return kNumRegFamilies + (slice_width_for(kb, forced) == kSliceWidths[0] ? 0 : 1);
+// Kernel family of bucket kB (kB <= kKbSliceMax).
+__host__ __device__ inline int nw_family_of(int kb, const NwMap &m) {
+  if (kb <= m.pk_top) {
+    int f = 0;
+    while (pk_cells(kb, m.pk_cap) > kPkFamilies[f].hi) ++f;
+    return kFirstPkFamily + f;
+  }
+  if (kb > kKbRegMax) return kNumRegFamilies + (slice_width_for(kb, m.forced) == kSliceWidths[0] ? 0 : 1);
   int f = 0;
   while (kb > kRegFamilies[f].hi) ++f;
   return f;
 }
 
 // Pairs one wave task of bucket kB covers in family f.
-__host__ __device__ inline int nw_pairs_per_wave(int kb, int f) {
+__host__ __device__ inline int nw_pairs_per_wave(int kb, int f, int pk_cap) {
+  if (f >= kFirstPkFamily) return 64 / pk_lanes(kb, pk_cap);
   return f >= kNumRegFamilies ? 64 / slice_lanes(kb, kSliceWidths[f - kNumRegFamilies]) : 64;
 }
 
@@ -73,6 +116,7 @@ struct NwPlan {
   uint2 list[kNumFamilies][kNumBuckets];
   uint32_t ntasks[kNumFamilies];
   uint32_t nbuckets[kNumFamilies];
+  uint32_t next[kNumFamilies];  // packed families: tasks taken past the first one of each block
 };
 
 struct NwFusedArgs {
@@ -81,8 +125,17 @@ struct NwFusedArgs {
   const int32_t *len;
   const int2 *pairs;
   const uint32_t *order;
-  const NwPlan *plan;
+  NwPlan *plan;
   float *out;
+};
+// A packed family's launch: one direction slot per block, the slice width cap,
+// and the read set's upper code bits (null when every read is ACGT only).
+struct PkLaunchArgs {
+  uint32_t *dirs;
+  int64_t words;  // per slot
+  int cap;
+  bool f16;  // every key of the family's buckets is at most kPkF16Top
+  const uint32_t *pack_hi;
 };
 
 // Each launcher runs `blocks` one-wave blocks of its family.
@@ -92,5 +145,9 @@ void launch_nw_reg_family2(hipStream_t s, unsigned blocks, const NwFusedArgs &a)
 void launch_nw_reg_family3(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
 void launch_nw_sliced_family24(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
 void launch_nw_sliced_family32(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
+void launch_nw_pk_family0(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k);
+void launch_nw_pk_family1(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k);
+void launch_nw_pk_family2(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k);
+void launch_nw_pk_family3(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k);
 
 }  // namespace crispy

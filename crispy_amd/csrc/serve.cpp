@@ -60,6 +60,7 @@ struct Job {
   int K = 6, band = 10;
   float kthr = 0.f, nthr = 0.f;
   int64_t est = 0;
+  int64_t scratch = 0;  // charged beside `est`: the NW directions' allowance
   int64_t held = 0;  // device bytes the slot's context held after the job
   // outgrew its charge while other jobs ran: queued again at the head,
   // charged the whole budget, so it runs alone
@@ -178,8 +179,11 @@ void worker_loop(crispy_server *srv, int slot) {
         if (!srv->queue.empty()) {
           // FIFO: the head job starts when it fits the budget next to what the
           // other slots hold
-          const int64_t held = srv->charge[slot];
-          const int64_t need = std::max(held, srv->queue.front()->est);
+          const int64_t held = srv->charge[slot], sheld = crispy_ctx_scratch_bytes(ctx);
+          const Job &head = *srv->queue.front();
+          // a job run again alone: one cap, the budget, over all its buffers
+          const int64_t scratch = head.solo ? 0 : std::max(sheld, head.scratch);
+          const int64_t need = head.solo ? std::max(held, head.est) : std::max(held - sheld, head.est) + scratch;
           if (srv->reserved - held + need <= srv->budget) {
             job = srv->queue.front();
             srv->queue.pop_front();
@@ -189,7 +193,8 @@ void worker_loop(crispy_server *srv, int slot) {
             srv->running += 1;
             if (!job->solo) job->t_start = Clock::now();
             // the job's buffers may not outgrow what it is charged
-            crispy_ctx_set_mem_limit(ctx, need);
+            crispy_ctx_set_mem_limit(ctx, need - scratch);
+            crispy_ctx_set_scratch_limit(ctx, job->solo ? -1 : scratch);
             break;
           }
           if (held > 0) {
@@ -220,6 +225,7 @@ void worker_loop(crispy_server *srv, int slot) {
         // whole budget, before the jobs behind it
         job->solo = true;
         job->est = srv->budget;
+        job->scratch = 0;
         job->status = CRISPY_OK;
         job->error.clear();
         srv->put_block(std::move(job->res));
@@ -355,8 +361,20 @@ int64_t crispy_server_submit(crispy_server *srv, const char *kmer_bases, const i
     }
   }
   job->est = crispy_server_job_bytes(job->kb(), job->koff.data(), n, K, band);
+  std::vector<int64_t> lens;
+  const auto &noff = job->same_reads ? job->koff : job->noff;
+  for (int32_t r = 0; r < n; ++r) lens.push_back(noff[r + 1] - noff[r]);
   std::lock_guard<std::mutex> lk(srv->mu);
   if (job->est > srv->budget) return CRISPY_ERR_NOMEM;  // would never be admitted
+  // What is left of an even share of the budget goes to the directions, so the
+  // slots still run side by side; 2 bits per band position and row.
+  {
+    const int64_t len = n > 0 ? *std::max_element(lens.begin(), lens.end()) : 0;
+    const int64_t kb = band >= 2 ? len / band : len;
+    const double want = 1.5 * std::min<double>((double)n * (n - 1) / 2, 256.0 * n) * (len + 32) * (2 * kb + 32) / 4;
+    const int64_t share = srv->budget / (int64_t)srv->ctxs.size() - job->est;
+    job->scratch = std::max<int64_t>(0, std::min<int64_t>({share, int64_t(4) << 30, (int64_t)std::min(want, 1e12)}));
+  }
   job->id = srv->next_id++;
   job->t_submit = Clock::now();
   srv->jobs[job->id] = job;
@@ -395,7 +413,7 @@ int crispy_server_job_times(crispy_server *srv, int64_t job_id, double *submit_m
   if (submit_ms) *submit_ms = ms(it->second->t_submit - t0).count();
   if (start_ms) *start_ms = ms(it->second->t_start - t0).count();
   if (end_ms) *end_ms = ms(it->second->t_end - t0).count();
-  if (est_bytes) *est_bytes = it->second->est;
+  if (est_bytes) *est_bytes = it->second->est + it->second->scratch;
   if (held_bytes) *held_bytes = it->second->held;
   return CRISPY_OK;
 }

@@ -65,6 +65,13 @@ int64_t crispy_ctx_device_bytes(const crispy_ctx *ctx);
  * them as they were.  No counterpart in the reference: the job server charges
  * each running job against its HBM budget with it. */
 int crispy_ctx_set_mem_limit(crispy_ctx *ctx, int64_t bytes);
+/* The NW directions' scratch (up to 4 GiB for large pair lists) counts within
+ * that cap by default (-1): the NW stage takes what is left of it, with a
+ * slower form when that is too little.  bytes >= 0 gives the scratch an
+ * allowance of its own beside the cap, as the job server does;
+ * crispy_ctx_scratch_bytes is what it holds.  No counterpart in the reference. */
+int crispy_ctx_set_scratch_limit(crispy_ctx *ctx, int64_t bytes);
+int64_t crispy_ctx_scratch_bytes(const crispy_ctx *ctx);
 /* Frees every device buffer of the context (reads, profiles, results); the
  * streams stay.  Buffers otherwise only grow, so a long-lived context holds
  * the largest job it has run. */
@@ -240,7 +247,7 @@ int crispy_nw_fetch_sorted(crispy_ctx *ctx, int64_t first, int64_t count, int32_
  * context's stream.  Query returns the summed duration (ms), the number of
  * launches and the algorithmic work units since the last reset:
  *   "kmer_profile" reads, "kmer_tile" read pairs evaluated (i < j),
- *   "nw_band_reg" and "nw_generic" in-band DP cells, "kmer_sort",
+ *   "nw_band_pk", "nw_band_reg", "nw_band_sliced" and "nw_generic" in-band DP cells, "kmer_sort",
  *   "nw_bucket", "nw_filter" elements. */
 int crispy_timing_enable(crispy_ctx *ctx, int enable);
 int crispy_timing_reset(crispy_ctx *ctx);
