@@ -35,13 +35,17 @@ constexpr int kGenericBucket = kKbSliceMax + 1;
 
 // k-mer tile geometry.
 constexpr int kTile = 128;        // reads per tile side
-constexpr int kChunkWords = 16;   // bitmap words staged in LDS per step (24 for 40- and 48-word bitmaps)
+constexpr int kChunkWords = 16;   // bitmap words staged in LDS per step of the tile kernel
 constexpr int kBitmapSlack = 32;  // words after the last bitmap row: a last chunk may be staged whole
 // Buckets of the hashed k = 6 candidate filter: 1,280, 1,536 or 2,048 (40,
 // 48 or 64 bitmap words per read, in 8-word groups); fewer buckets mean less
 // tile work and more candidates for the exact passes.
 constexpr int kHashWordsMax = 64;
 __host__ __device__ constexpr bool valid_hash_words(int w) { return w == 40 || w == 48 || w == 64; }
+// Bucket bitmaps of 40 and 48 words are stored by blocks of kTile reads, in
+// 16-byte pieces: piece p of every read of the block, then piece p + 1 (the
+// sweep kernel reads whole runs); 64-word ones read by read.
+__host__ __device__ constexpr bool hash_blocked(int w) { return w < 64; }
 // The candidate tiles append to kCandSegs output segments, each with its own
 // counter kSegStride u64 words (4 KB) from the next: one counter for the
 // whole chip serialises the per-wave reservations (~600k atomics per
@@ -124,7 +128,7 @@ struct KmerState {
   // k = 6 candidate filter: presence of the 4,096 codes hashed into
   // 32 x hash_words buckets, and T - (distinct buckets); `hashed` when the
   // profile holds them.  hash_buckets: the setting (0 = default).
-  DevBuf hbitmap, hexcess;
+  DevBuf hbitmap, hexcess, hbound;  // hbound: the sweep's bound G per read (kmer.hip)
   bool hashed = false;
   int hash_words = crispy::kHashWordsMax;
   int hash_buckets = 0;

@@ -217,7 +217,10 @@ __global__ __launch_bounds__(128) void kmer_profile_kernel(
   if (HASH) {  // the barrier after the scan ordered the bucket bits before these reads
     if (tid < HW) {
       const uint32_t w = hbm[tid];
-      hbitmap[(int64_t)r * HW + tid] = w;
+      if constexpr (hash_blocked(HW))
+        hbitmap[((int64_t)(r / kTile) * (HW / 4) + tid / 4) * (4 * kTile) + r % kTile * 4 + tid % 4] = w;
+      else
+        hbitmap[(int64_t)r * HW + tid] = w;
       atomicAdd(&s_hdistinct, __popc(w));
     }
     __syncthreads();
@@ -284,7 +287,9 @@ constexpr int kCandPopShift = 44;
 constexpr int kCandWin = 32;
 constexpr int kListSlack = 32;
 static_assert(kCandWin % 4 == 0 && kCandWin <= kListSlack, "a window starts on a word at or before the list's last code");
-// Pairs from which the K <= 6 exact counts run as a pass of their own (auto mode).
+// Pairs from which the K <= 6 exact counts run as a pass of their own (auto
+// mode): k = 6 (hashed sweep), and K < 6 (tiles on the exact bitmaps).
+constexpr int64_t kExactPassPairs6 = 400000000;
 constexpr int64_t kExactPassPairs = 1000000000;
 constexpr uint64_t kCandKeyMask = (1ull << 40) - 1;
 
@@ -403,7 +408,7 @@ __device__ __forceinline__ int wave_incl_sum(int v, int lane) {
   return v;
 }
 
-template <int WP, bool CAND, int CW = kChunkWords>
+template <int WP, bool CAND>
 __global__ __launch_bounds__(128, 2) void kmer_tile_mfma_kernel(
     const uint32_t *__restrict__ bitmap, const int32_t *__restrict__ Tn,
     const int32_t *__restrict__ rcnt, const int64_t *__restrict__ roff,
@@ -412,13 +417,9 @@ __global__ __launch_bounds__(128, 2) void kmer_tile_mfma_kernel(
     unsigned long long *__restrict__ counter, uint64_t *__restrict__ out_keys,
     float *__restrict__ out_dists, int64_t cap) {
   static_assert(WP % 8 == 0 && WP <= 128, "bitmap tiles hold at most 4,096 presence bits, in 8-word groups");
-  // chunks of CW words (16, or 24 for 40- and 48-word bitmaps: 2 chunks, 2
-  // barrier pairs per tile); the last chunk may hold fewer 8-word groups (the
-  // rest of it, read past the row, is staged but not used: the bitmap buffers
-  // end with kBitmapSlack words of slack)
-  static_assert(CW == 16 || CW == 24, "16- or 24-word chunks");
-  constexpr int NCH = (WP + CW - 1) / CW;
-  constexpr int kLastGroups = (WP - (NCH - 1) * CW) / 8;  // 8-word groups in the last chunk
+  constexpr int CW = kChunkWords;
+  static_assert(WP % CW == 0, "whole chunks");
+  constexpr int NCH = WP / CW;
   constexpr int kRow = CW + 4;  // padded row stride of a staged chunk (words)
   constexpr int kStageWords = 2 * kTile * kRow;
   __shared__ uint32_t Ps[kStageWords];  // bitmap chunk in the main loop, then repeat lists
@@ -446,14 +447,13 @@ __global__ __launch_bounds__(128, 2) void kmer_tile_mfma_kernel(
   const int g = lane >> 5, r32 = lane & 31;
 
   // loader: a chunk is CW words of each of the 256 reads.  TPR lanes share a
-  // read, each loading UPT 16-byte pieces of it (16-word chunks: lane quads,
-  // one piece each; 24-word chunks: lane pairs, three each), so a wave
-  // instruction reads whole runs; the block's 128 lanes cover RP reads of the
+  // read, each loading UPT 16-byte pieces of it, so a wave instruction reads
+  // whole runs; the block's 128 lanes cover RP reads of the
   // rows and of the columns per pass, NPASS passes.  Rows past n load read 0
   // (always valid): their pairs are masked in the epilogue.  Chunk 0 is
   // requested first and the per-read data right after it, so their
   // latencies overlap.
-  constexpr int TPR = CW == 16 ? 4 : 2, UPT = CW / 4 / TPR;
+  constexpr int TPR = 4, UPT = CW / 4 / TPR;
   constexpr int RP = 128 / TPR, NPASS = kTile / RP;
   constexpr int NLD = NPASS * UPT;  // 16-byte pieces per lane per side
   const int lq = tid % TPR, lr = tid / TPR;
@@ -564,7 +564,6 @@ __global__ __launch_bounds__(128, 2) void kmer_tile_mfma_kernel(
     }
 #pragma unroll
     for (int m = 0; m < CW / 8; ++m) {  // 8-word groups
-      if (ch == NCH - 1 && m >= kLastGroups) break;  // block-uniform
       uint4 xa[2], xb[4];
 #pragma unroll
       for (int fa = 0; fa < 2; ++fa)
@@ -848,6 +847,272 @@ __global__ __launch_bounds__(128, 2) void kmer_tile_mfma_kernel(
     });
     qcount += qn;
   });
+  if (qcount > 0) flush();
+}
+
+// ------------------------------------------------- hashed candidate sweep
+// The candidate form on bucket bitmaps of WP words (hash_blocked): a wave keeps
+// 64 rows (their raw words in registers) and sweeps `1 << sweep_log` column
+// tiles of a super-tile with no barrier and no LDS staging: the 4 column
+// operands of the next 8-word group are loaded, whole cache lines, while the
+// current group's 32 MFMAs run (the 4 waves of a block, 256 rows, sweep the
+// same columns, mostly out of the same L1).  MFMA, bit planes and bound are the
+// tile kernel's; survivors stay queued in LDS across the sweep as row quads
+// and are told apart at the flush, a lane each (one flush per wave, mostly).
+//
+// What bounds it: the matrix pipe needs 4 WP MFMAs x 32 cycles per wave and
+// tile (160 at 40 words); the loop with its ~5 bit-plane instructions per MFMA
+// and the bound tests runs at ~43 cycles per MFMA and SIMD without survivors
+// (part of it the clock, which dense operands pull below 2.4 GHz), ~50 with
+// 3 survivors per wave and tile.  Measured against the tile kernel (a block
+// per 128 x 128 tile: 4 barriers, a cold start and an atomic round trip per
+// tile) at 40 words: 3.1e10 pairs of 400-900 bp 15.7 -> 12.6 ms, 5e9 pairs of
+// 150-550 bp 2.89 -> 2.36 ms.  The same sweep with the columns copied to LDS
+// (double buffer, one barrier per tile) took 13.5 ms where this took 13.2.
+//
+// Unit u of a launch: row pair u % 8 of a super-tile (8 blocks next to each
+// other sweep the same columns), then the column group, then the super-tile.
+// Slots outside [slot0, slot0 + nslots), below the diagonal or past the last
+// tile are left out of a wave's columns.
+constexpr int kSweepQueue = 640;  // entries per wave
+// Rounds of resident blocks (2 per CU) that a launch has at least before its
+// sweeps get longer (8 against 2: 30,000 to 60,000 reads 0.1 to 4 % faster).
+constexpr int kSweepRounds = 8;
+
+// G per read (see the tile kernel) for n reads, padded to whole tiles with a
+// bound that is never the smaller one, and the candidate segments' counters
+// zeroed.
+__global__ __launch_bounds__(256) void kmer_bound_kernel(const int32_t *__restrict__ Tn,
+                                                         const int32_t *__restrict__ excess, int32_t n, int npad,
+                                                         float cut, int tshift, float *__restrict__ G,
+                                                         unsigned long long *__restrict__ seg) {
+  static_assert(kCandSegs <= 256, "block 0 zeroes every counter");
+  if (blockIdx.x == 0 && threadIdx.x < kCandSegs) seg[(size_t)threadIdx.x * kSegStride] = 0ull;
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= npad) return;
+  float g = 3e38f;
+  if (r < n) g = fmaxf(fmaf((float)(Tn[r] - tshift), cut, -1.0f) - (float)excess[r], 0.0f);
+  G[r] = g;
+}
+
+template <int WP>
+__global__ __launch_bounds__(256, 2) void kmer_sweep_kernel(
+    const uint32_t *__restrict__ bits, const float *__restrict__ G, int32_t n, int nb, int64_t slot0, int64_t nslots,
+    int64_t units, int64_t per_xcd, int sweep_log, int kshift, unsigned long long *__restrict__ counter,
+    uint64_t *__restrict__ out_keys, int64_t cap) {
+  static_assert(hash_blocked(WP) && WP % 8 == 0, "blocked bitmaps of whole 8-word groups");
+  constexpr int NG = WP / 8;  // 8-word groups
+  __shared__ __align__(16) float sG[4][64];
+  __shared__ uint2 sQ[4][kSweepQueue];
+
+  const int64_t bid = blockIdx.x;
+  const int64_t u = (bid & 7) * per_xcd + (bid >> 3);
+  if (u >= units) return;
+  const int glog = 4 - sweep_log;
+  const int64_t super = slot0 / kSuperSlots + (u >> (3 + glog));
+  const int pr = (int)(u & 7), cg = (int)(u >> 3) & ((1 << glog) - 1);
+  const int ns = (nb + kSuperTiles - 1) / kSuperTiles;
+  int I, J;
+  tile_coords(super, ns, I, J);
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 5, r32 = lane & 31;
+  const int br = 2 * pr + (wv >> 1);  // the wave's tile row in the super-tile, rows 64 (wv & 1) .. + 63 of it
+  const int bi = I * kSuperTiles + br;
+  if (bi >= nb) return;
+  // its column tiles: the group's, on or right of the diagonal, in the slot range
+  const int64_t s0 = super * kSuperSlots + br * kSuperTiles;
+  int c = max(cg << sweep_log, (int)min(max(slot0 - s0, (int64_t)0), (int64_t)kSuperTiles));
+  if (I == J) c = max(c, br);
+  const int c1 = min(min((cg + 1) << sweep_log, nb - J * kSuperTiles),
+                     (int)min(max(slot0 + nslots - s0, (int64_t)0), (int64_t)kSuperTiles));
+  if (c >= c1) return;
+
+  // 16-byte pieces: (piece, read) of tile b at pieces[(b * WP / 4 + piece) * kTile + read]
+  const uint4 *pieces = reinterpret_cast<const uint4 *>(bits);
+  auto ld = [](const uint4 *at) {
+    const uint4 v = *at;
+    return make_uint4(v.x, v.y, v.z, v.w);
+  };
+  const uint4 *cols = pieces + (int64_t)J * kSuperTiles * (WP / 4) * kTile + g * kTile + r32;
+  auto ldcol = [&](int col, int m, int fb) { return ld(cols + (col * (WP / 4) + 2 * m) * kTile + fb * 32); };
+  uint4 xb[4];
+#pragma unroll
+  for (int fb = 0; fb < 4; ++fb) xb[fb] = ldcol(c, 0, fb);
+  uint4 xa[2][NG];  // the wave's rows
+#pragma unroll
+  for (int fa = 0; fa < 2; ++fa)
+#pragma unroll
+    for (int m = 0; m < NG; ++m)
+      xa[fa][m] = ld(pieces + ((int64_t)bi * (WP / 4) + 2 * m + g) * kTile + (wv & 1) * 64 + fa * 32 + r32);
+  const int row0 = bi * kTile + (wv & 1) * 64, col0 = J * kSuperTiles * kTile;
+  sG[wv][lane] = G[row0 + lane];
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  uint32_t gq[2][4], grmin[2];  // smallest bound of each of the lane's row quads 4g + 8q .. + 3, and of all of them
+#pragma unroll
+  for (int fa = 0; fa < 2; ++fa) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const lds_f4 v = *reinterpret_cast<const lds_f4 *>(&sG[wv][fa * 32 + 4 * g + 8 * q]);
+      gq[fa][q] = min(min(__float_as_uint(v[0]), __float_as_uint(v[1])), min(__float_as_uint(v[2]), __float_as_uint(v[3])));
+    }
+    grmin[fa] = min(min(gq[fa][0], gq[fa][1]), min(gq[fa][2], gq[fa][3]));
+  }
+
+  // Queue entry: a lane's 4 popcounts of a row quad (11 bits each) and
+  // quad << 11 | column in the super-tile; the pairs are told apart at the
+  // flush, one entry per lane.
+  static_assert(WP * 32 < 2048, "popcounts of 11 bits");
+  uint2 *queue = sQ[wv];
+  int qcount = 0;  // wave-uniform
+  auto flush = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    // one of the XCD's 32 segments (the refine pass reads them on the same XCD,
+    // and an XCD's units share their reads) by a multiplicative hash of the
+    // unit, wave and column: near the diagonal lie more candidates
+    static_assert(kCandSegs == 256, "8 XCDs, 5 hash bits");
+    const uint32_t seg = ((uint32_t)(u * 64 + wv * 16 + (c & 15)) * 2654435761u) >> 27 << 3 | (uint32_t)(bid & 7);
+    uint64_t *out = out_keys + (size_t)seg * cap;
+    for (int e = 0; e < qcount; e += 64) {
+      const bool have = e + lane < qcount;
+      const uint2 x = queue[have ? e + lane : 0];
+      const uint32_t id = x.x >> 22 | (x.y >> 22) << 10;
+      const int row = 4 * (int)(id >> 11), j = col0 + (int)(id & 2047u);
+      const uint32_t pop[4] = {x.x & 2047u, x.x >> 11 & 2047u, x.y & 2047u, x.y >> 11 & 2047u};
+      const lds_f4 gr = *reinterpret_cast<const lds_f4 *>(&sG[wv][row]);
+      const float gj = G[j];
+      uint64_t ball[4];
+      int total = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {  // popcount >= min(G_i, G_j): the pair may pass
+        ball[t] = __ballot(have && row0 + row + t < j && j < n && (float)pop[t] >= fminf(gr[t], gj));
+        total += __popcll(ball[t]);
+      }
+      unsigned long long base = 0;
+      if (lane == 0 && total) base = atomicAdd(counter + (size_t)seg * kSegStride, (unsigned long long)total);
+      int64_t pos = (int64_t)__shfl(base, 0, 64);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int64_t at = pos + __builtin_amdgcn_mbcnt_hi((uint32_t)(ball[t] >> 32),
+                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)ball[t], 0u));
+        if ((ball[t] >> lane & 1) && at < cap)
+          out[at] = ((uint64_t)(row0 + row + t) << kshift) | (uint64_t)j | ((uint64_t)pop[t] << kCandPopShift);
+        pos += __popcll(ball[t]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    qcount = 0;
+  };
+
+  // the planes' masks in scalar registers: as literals they double the ANDs' size
+  uint32_t mask[3] = {0x11111111u, 0x22222222u, 0x44444444u};
+  asm volatile("" : "+s"(mask[0]), "+s"(mask[1]), "+s"(mask[2]));
+  for (; c < c1; ++c) {
+    const int bj = J * kSuperTiles + c;
+    // values made opaque here, or the compiler keeps the rows' bit planes in
+    // registers across the sweep and spills
+#pragma unroll
+    for (int fa = 0; fa < 2; ++fa)
+#pragma unroll
+      for (int m = 0; m < NG; ++m)
+        asm volatile("" : "+v"(xa[fa][m].x), "+v"(xa[fa][m].y), "+v"(xa[fa][m].z), "+v"(xa[fa][m].w));
+    mfma_v16f acc[2][4];
+    uint32_t gc[4];
+    auto ext = [&](const uint4 &x, int pl) {  // bit plane pl as FP4 (see the tile kernel)
+      const uint32_t M = pl == 3 ? mask[1] : mask[pl];
+      const int sh = pl < 3 ? 0 : 2;
+      mfma_v8i e;
+      e[0] = (int)((x.x >> sh) & M);
+      e[1] = (int)((x.y >> sh) & M);
+      e[2] = (int)((x.z >> sh) & M);
+      e[3] = (int)((x.w >> sh) & M);
+      e[4] = e[5] = e[6] = e[7] = 0;  // unused by FP4 operands
+      return e;
+    };
+    static_for<NG>([&](auto MG) {
+      constexpr int m = decltype(MG)::value;
+      uint4 xn[4];  // the next group's columns (after the last tile: the last tile's again)
+#pragma unroll
+      for (int fb = 0; fb < 4; ++fb)
+        xn[fb] = m + 1 < NG ? ldcol(c, m + 1, fb) : ldcol(min(c + 1, c1 - 1), 0, fb);
+      if constexpr (m == NG - 1) {
+#pragma unroll
+        for (int fb = 0; fb < 4; ++fb) gc[fb] = __float_as_uint(G[bj * kTile + fb * 32 + r32]);
+      }
+      mfma_v8i ea[2], en[2], eb[4];
+#pragma unroll
+      for (int fa = 0; fa < 2; ++fa) ea[fa] = ext(xa[fa][m], 0);
+#pragma unroll
+      for (int fb = 0; fb < 4; ++fb) eb[fb] = ext(xb[fb], 0);
+      static_for<4>([&](auto PL) {
+        constexpr int pl = decltype(PL)::value;
+        constexpr int scale = pl < 3 ? kUnitScale + 2 - 2 * pl : kUnitScale;
+        static_for<4>([&](auto FB) {
+          constexpr int fb = decltype(FB)::value;
+#pragma unroll
+          for (int fa = 0; fa < 2; ++fa) {
+            mfma_v16f z;
+            if constexpr (m == 0 && pl == 0)
+              z = (mfma_v16f)(0.0f);
+            else
+              z = acc[fa][fb];
+            acc[fa][fb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ea[fa], eb[fb], z, kFp4, kFp4, 0, scale, 0,
+                                                                          kUnitScale);
+          }
+          if constexpr (pl < 3) {
+            eb[fb] = ext(xb[fb], pl + 1);
+            if constexpr (fb >= 2) en[fb - 2] = ext(xa[fb - 2][m], pl + 1);
+          }
+        });
+        if constexpr (pl < 3) {
+          ea[0] = en[0];
+          ea[1] = en[1];
+        }
+      });
+#pragma unroll
+      for (int fb = 0; fb < 4; ++fb) xb[fb] = make_uint4(xn[fb].x, xn[fb].y, xn[fb].z, xn[fb].w);
+      __builtin_amdgcn_sched_barrier(0);  // or every group's column reads come first, and spill
+    });
+
+    // every product is complete here (the compiler would sink a fragment's
+    // MFMAs past the branches of the fragments before it, and spill)
+#pragma unroll
+    for (int fa = 0; fa < 2; ++fa)
+#pragma unroll
+      for (int fb = 0; fb < 4; ++fb) asm volatile("" : "+v"(acc[fa][fb]));
+    // the bound: a fragment's largest value first (most fragments of a large
+    // run keep nothing), then each row quad's
+    static_for<2>([&](auto FA) {
+      constexpr int fa = decltype(FA)::value;
+      static_for<4>([&](auto FB) {
+        constexpr int fb = decltype(FB)::value;
+        uint32_t amq[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          amq[q] = max(max(__float_as_uint(acc[fa][fb][4 * q]), __float_as_uint(acc[fa][fb][4 * q + 1])),
+                       max(__float_as_uint(acc[fa][fb][4 * q + 2]), __float_as_uint(acc[fa][fb][4 * q + 3])));
+        const uint32_t amax = max(max(amq[0], amq[1]), max(amq[2], amq[3]));
+        if (__ballot(amax >= min(grmin[fa], gc[fb])) == 0) return;  // wave-uniform
+        if (qcount > kSweepQueue - 256) flush();
+        static_for<4>([&](auto Q) {
+          constexpr int q = decltype(Q)::value;
+          const bool hit = amq[q] >= min(gq[fa][q], gc[fb]);
+          const uint64_t ball = __ballot(hit);
+          if (ball == 0) return;  // wave-uniform
+          if (hit) {  // slot: the kept lanes below this one
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(ball >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)ball, 0u));
+            const uint32_t id = (uint32_t)((fa * 8 + 2 * q + g) << 11) | (uint32_t)(c * kTile + fb * 32 + r32);
+            queue[qcount + (int)below] =
+                make_uint2((uint32_t)acc[fa][fb][4 * q] | (uint32_t)acc[fa][fb][4 * q + 1] << 11 | id << 22,
+                           (uint32_t)acc[fa][fb][4 * q + 2] | (uint32_t)acc[fa][fb][4 * q + 3] << 11 | (id >> 10) << 22);
+          }
+          qcount += __popcll(ball);
+        });
+      });
+    });
+  }
+  --c;
   if (qcount > 0) flush();
 }
 
@@ -1373,16 +1638,20 @@ static int launch_tiles(crispy_ctx *ctx, int32_t n, int nb, int64_t tb, int64_t 
   constexpr bool HASHED = HW > 0;
   static_assert(!HASHED || (K == 6 && CAND), "the hashed filter is the k = 6 candidate form");
   constexpr int WP = HASHED ? HW : kmer_words(K);
-  constexpr int CW = CAND && (WP == 40 || WP == 48) ? 24 : kChunkWords;  // chunk words (2 chunks per tile)
+  constexpr bool SWEEP = HASHED && hash_blocked(WP);
   KmerState &km = ctx->km;
   const DevBuf &bits = HASHED ? km.hbitmap : km.bitmap;
   const DevBuf &excess = HASHED ? km.hexcess : km.excess;
-  const int64_t per_xcd = (nt + 7) / 8;
-  const int64_t grid = per_xcd * 8;
   const float cut = 1.0f - thr - 2e-5f;
   uint32_t thr_bits;
   std::memcpy(&thr_bits, &thr, sizeof thr_bits);
   unsigned long long *counter = CAND ? km.seg.as<unsigned long long>() : km.counter.as<unsigned long long>();
+  // sweep: the longest that still leaves kSweepRounds rounds of resident blocks
+  const int64_t supers = (tb + nt - 1) / kSuperSlots - tb / kSuperSlots + 1;
+  int sweep_log = 4;
+  while (sweep_log > 0 && supers * 8 << (4 - sweep_log) < (int64_t)kSweepRounds * 2 * ctx->cus) --sweep_log;
+  const int64_t units = supers * 8 << (4 - sweep_log);
+  if (SWEEP) CRISPY_TRY(ensure(ctx, km.hbound, sizeof(float) * (size_t)nb * kTile));
   hipEvent_t ev;
   timer_begin(ctx, "kmer_tile", &ev);
   CRISPY_TRY(run_segment(
@@ -1390,18 +1659,30 @@ static int launch_tiles(crispy_ctx *ctx, int32_t n, int nb, int64_t tb, int64_t 
       {(uintptr_t)WP, (uintptr_t)CAND, (uintptr_t)bits.p, (uintptr_t)km.T.p, (uintptr_t)km.rcnt.p,
        (uintptr_t)km.roffc.p, (uintptr_t)km.rlistc.p, (uintptr_t)excess.p, (uintptr_t)n, (uintptr_t)nb,
        (uintptr_t)tb, (uintptr_t)nt, thr_bits, (uintptr_t)tshift, (uintptr_t)km.kshift, (uintptr_t)counter,
-       (uintptr_t)km.seg_stat.p, (uintptr_t)out_keys, (uintptr_t)out_dists, (uintptr_t)cap},
+       (uintptr_t)km.seg_stat.p, (uintptr_t)out_keys, (uintptr_t)out_dists, (uintptr_t)cap, (uintptr_t)km.hbound.p},
       "k-mer tile pass", [&](bool) -> int {
-        if (CAND)
-          zero_segs_kernel<<<1, kCandSegs, 0, ctx->stream>>>(counter);
-        else
-          zero_counter_kernel<<<1, 1, 0, ctx->stream>>>(counter);
-        CRISPY_LAUNCHED(ctx);
-        kmer_tile_mfma_kernel<WP, CAND, CW><<<(unsigned)grid, 128, 0, ctx->stream>>>(
-            bits.as<uint32_t>(), km.T.as<int32_t>(), km.rcnt.as<int32_t>(), km.roffc.as<int64_t>(),
-            km.rlistc.as<uint32_t>(), excess.as<int32_t>(), n, nb, tb, nt, per_xcd, thr, cut, tshift,
-            km.kshift, counter, out_keys, out_dists, cap);
-        CRISPY_LAUNCHED(ctx);
+        if constexpr (SWEEP) {
+          kmer_bound_kernel<<<(nb * kTile + 255) / 256, 256, 0, ctx->stream>>>(
+              km.T.as<int32_t>(), excess.as<int32_t>(), n, nb * kTile, cut, tshift, km.hbound.as<float>(), counter);
+          CRISPY_LAUNCHED(ctx);
+          const int64_t per_xcd = (units + 7) / 8;
+          kmer_sweep_kernel<WP><<<(unsigned)(per_xcd * 8), 256, 0, ctx->stream>>>(
+              bits.as<uint32_t>(), km.hbound.as<float>(), n, nb, tb, nt, units, per_xcd, sweep_log, km.kshift, counter,
+              out_keys, cap);
+          CRISPY_LAUNCHED(ctx);
+        } else {
+          if (CAND)
+            zero_segs_kernel<<<1, kCandSegs, 0, ctx->stream>>>(counter);
+          else
+            zero_counter_kernel<<<1, 1, 0, ctx->stream>>>(counter);
+          CRISPY_LAUNCHED(ctx);
+          const int64_t per_xcd = (nt + 7) / 8;
+          kmer_tile_mfma_kernel<WP, CAND><<<(unsigned)(per_xcd * 8), 128, 0, ctx->stream>>>(
+              bits.as<uint32_t>(), km.T.as<int32_t>(), km.rcnt.as<int32_t>(), km.roffc.as<int64_t>(),
+              km.rlistc.as<uint32_t>(), excess.as<int32_t>(), n, nb, tb, nt, per_xcd, thr, cut, tshift,
+              km.kshift, counter, out_keys, out_dists, cap);
+          CRISPY_LAUNCHED(ctx);
+        }
         if (CAND) {
           seg_stat_kernel<<<1, kCandSegs, 0, ctx->stream>>>(counter, km.seg_stat.as<unsigned long long>());
           CRISPY_LAUNCHED(ctx);
@@ -1458,8 +1739,8 @@ static int build_profiles(crispy_ctx *ctx, int KP, int K, bool hash) {
   CRISPY_TRY(ensure(ctx, km.rcnt, sizeof(int32_t) * (n + 1)));
   CRISPY_TRY(ensure(ctx, km.excess, sizeof(int32_t) * (n + 1)));
   if (km.hashed) {
-    // + kBitmapSlack: the tile's last part-filled chunk is staged whole
-    CRISPY_TRY(ensure(ctx, km.hbitmap, sizeof(uint32_t) * ((size_t)n * km.hash_words + kBitmapSlack)));
+    // whole blocks of kTile reads (hash_blocked)
+    CRISPY_TRY(ensure(ctx, km.hbitmap, sizeof(uint32_t) * ((size_t)(n + kTile - 1) / kTile * kTile * km.hash_words)));
     CRISPY_TRY(ensure(ctx, km.hexcess, sizeof(int32_t) * (n + 1)));
   }
   CRISPY_TRY(ensure(ctx, km.roff, sizeof(int64_t) * (n + 1)));
@@ -1723,13 +2004,15 @@ int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
   while ((1 << km.kshift) < n) ++km.kshift;
   const int KP = K <= 6 ? K : 6;
   // K <= 6: exact counts in the tile, or in a pass of their own over the
-  // tile's candidates.  Measured on MI355X: the lean candidate tile plus the
-  // pass wins from ~10^9 pairs up (reads100k 9.8 -> 9.1 ms, reads250k 50.2
-  // -> 44.0 ms per k-mer run); below, the pass's latency-bound merges cost more
-  // than the tile saves (reads20k 0.78 -> 0.97 ms).  The candidate tiles of
-  // k = 6 run on the hashed bitmaps (half the words).
+  // tile's candidates.  Measured per k-mer run at k = 6, 150-550 bp, counts in
+  // the tile against the hashed sweep and the pass: 12,000 reads 0.48 and
+  // 0.66 ms, 20,000 0.78 and 0.87, 30,000 1.28 and 1.19, 45,000 2.34 and
+  // 1.71, 60,000 3.87 and 2.31; below, the extra passes' launches and
+  // latency-bound merges cost more than the sweep saves.  K < 6 runs its
+  // candidate tiles on the exact bitmaps, which win from ~10^9 pairs up.
   // exact_pass 2: the candidate form on the exact bitmaps (no hashing).
-  const bool separate = km.exact_pass >= 1 || (km.exact_pass == -1 && (int64_t)n * (n - 1) / 2 >= kExactPassPairs);
+  const bool separate = km.exact_pass >= 1 || (km.exact_pass == -1 &&
+                         (int64_t)n * (n - 1) / 2 >= (K == 6 ? kExactPassPairs6 : kExactPassPairs));
   CRISPY_TRY(build_profiles(ctx, KP, K, (K > 6 || separate) && km.exact_pass != 2));
   // the k = 6 candidate tiles: on the hashed bitmaps, or on the exact ones
   const TileFn tiles6 = !km.hashed                          ? launch_tiles<6, true>

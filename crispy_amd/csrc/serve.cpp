@@ -250,6 +250,8 @@ void worker_loop(crispy_server *srv, int slot) {
 // Widest half band kB = (L1 + L2) / (2 band) the register and sliced NW
 // kernels take (64 lanes x 24 cells per pair); wider pairs use the generic one.
 constexpr int64_t kSlicedMaxHalfBand = (64 * 24 - 1) / 2;
+// K = 6 jobs of this many pairs take hashed candidates (kExactPassPairs6 in kmer.hip).
+constexpr int64_t kCandidatePairs = 400000000;
 
 int64_t words_per_read(int K) {
   const int KP = K <= 6 ? K : 6;
@@ -287,9 +289,9 @@ int64_t crispy_server_job_bytes(const char *bases, const int64_t *offsets, int32
   const int64_t pairs = std::min<int64_t>(all_pairs, 256 * (int64_t)n);
   const int64_t reads = 2 * (nbases + nbases / 4 + 48 * (int64_t)n);
   int64_t prof = (int64_t)n * (4 * words_per_read(K) + 48) + 6 * nbases;
-  // K > 6: K-mer lists, the hashed k = 6 bitmaps (at most 2,048 bits) and their
-  // excess, candidates + their refined copy, the 256 x 4 KB segment counters
-  if (K > 6) prof += 2 * nbases + 16 * (int64_t)n + 260 * (int64_t)n + 16 * (std::max(guess, pairs) + 256) + (1 << 20);
+  // K > 6, and large K = 6 jobs: K-mer lists, the hashed k = 6 bitmaps (at most
+  // 2,048 bits) and their excess and bounds, candidates + their refined copy, the 256 x 4 KB segment counters
+  if (K > 6 || (K == 6 && all_pairs >= kCandidatePairs)) prof += 2 * nbases + 16 * (int64_t)n + 260 * (int64_t)n + 16 * (std::max(guess, pairs) + 256) + (1 << 20);
   int64_t est = reads + prof + 12 * guess + 72 * pairs + (int64_t)(8 << 20);
   const bool generic = band <= 1 || !clean || (band > 0 && maxlen / band > kSlicedMaxHalfBand);
   if (generic) est += 8 * std::min<int64_t>(pairs, 32768) * (maxlen + 1);
