@@ -187,7 +187,16 @@ __device__ __forceinline__ void nw_pk_wave(const uint32_t *__restrict__ pack, co
   // virtual lane W / C), where the last real cell has no "left"
   const uint32_t first_mask = g > 0 ? ~0u : 0u, last_mask = is_end ? 0u : ~0u;
   const int dead_v = W / C, dead_k = W - dead_v * C;
-  const uint32_t dead_mask = g != dead_v >> 1 ? ~0u : dead_v & 1 ? 0x0000FFFFu : 0xFFFF0000u;
+  // (its lanes by execution mask and its cell by masks in scalar registers: a
+  // vector mask was spilled, and its reload in every step waited for the
+  // direction stores; choosing the cell by branches moved the row's registers)
+  const bool dead_lane = g == dead_v >> 1;
+  const uint32_t dead_half = dead_v & 1 ? 0x0000FFFFu : 0xFFFF0000u;
+  uint32_t dead_near[4];  // cells C - 1, - 3, - 5, - 7: where W / (2 G) leaves it mostly
+#pragma unroll
+  for (int o = 0; o < 4; ++o)
+    dead_near[o] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(C - dead_k == 2 * o + 1 ? dead_half : ~0u));
+  const bool dead_far = (C - dead_k) % 2 == 0 || C - dead_k > 7;
 
   // row 0: M 0 at every position (positions with j < 0 are computed but never
   // read by a cell of the matrix: the boundary cells are set below)
@@ -201,12 +210,17 @@ __device__ __forceinline__ void nw_pk_wave(const uint32_t *__restrict__ pack, co
     Kv[k] = b + 0x00010001u * (44u + rank_left);
   }
   auto mask_dead = [&]() {
-    if (G == 1) {  // wave-uniform; then 2 C = W + 1
-      Kv[C - 1] &= 0x0000FFFFu;
-    } else {
+    if (dead_lane)
+      static_for_pk<0, 4>([&](auto O) {
+        constexpr int k = C - 1 - 2 * decltype(O)::value;
+        if constexpr (k >= 0) Kv[k >= 0 ? k : 0] &= dead_near[decltype(O)::value];
+      });
+    if (dead_far) {  // wave-uniform
+      asm volatile("");  // a branch, not selects in every step
       static_for_pk<0, C>([&](auto K) {
         constexpr int k = decltype(K)::value;
-        if (k == dead_k) Kv[k] &= dead_mask;  // wave-uniform
+        if constexpr ((C - k) % 2 == 0 || C - k > 7)
+          if (dead_lane) Kv[k] &= k == dead_k ? dead_half : ~0u;
       });
     }
   };
@@ -332,7 +346,7 @@ __device__ __forceinline__ void nw_pk_wave(const uint32_t *__restrict__ pack, co
         if (ihi == 0) Kv[0] = (Kv[0] & 0x0000FFFFu) | (kv0_old & 0xFFFF0000u);
       }
       // the left neighbour reads it in this step
-      if (dead_k == 0) Kv[0] &= dead_mask;  // wave-uniform
+      if (dead_k == 0 && dead_lane) Kv[0] &= dead_half;
     }
     // "left" of the last cells: the high half's first offer for the low half,
     // the next lane's low half's for the high half
