@@ -400,10 +400,10 @@ static int64_t family_grid(int f, int64_t np, int kb_lo, int kb_hi, const NwMap 
 }
 
 // The packed families' part of one DP phase: which kB they take, and per
-// family the blocks (= direction slots) and their scratch.
+// family the waves (= direction slots) and their scratch.
 struct PkPlan {
   NwMap map;
-  unsigned blocks[kNumPkFamilies] = {};
+  unsigned slots[kNumPkFamilies] = {};
   PkLaunchArgs args[kNumPkFamilies] = {};
   int64_t region[kNumWorkers] = {};  // scratch bytes of each worker stream: its families run one after the other
   int64_t bytes() const {
@@ -454,17 +454,27 @@ static double pk_plan_cap(int cus, int64_t np, int band, int maxlen, int kb_lo, 
     total += pairs / (64 / lanes) * task;
     longest = std::max(longest, task);
   }
+  // Blocks of four waves, one per SIMD, where up to two families run: one-wave
+  // blocks land unevenly (2,747 tasks put 2 to 4 on a SIMD, and the call ended
+  // with those of 4): 20,000 pairs of 1.1-1.5 kbp 2.61 -> 2.22 ms, a step with
+  // 0.84 M pairs of 200-300 bp 3.57 -> 3.50.  With more families at once, of
+  // several register counts, single waves fill the SIMDs better: 3.3 M pairs
+  // of 150-550 bp, four families, 17.0 ms for 17.6.
+  int families = 0;
+  for (const PkLaunchArgs &x : p.args) families += x.words > 0;
+  for (PkLaunchArgs &x : p.args) x.block_waves = families <= 2 ? kPkBlockWaves : 1;
   int64_t full = 0;
   for (int pass = 0; pass < 2; ++pass) {
     int64_t slots = 0;
     for (int64_t &r : p.region) r = 0;
     for (int f = 0; f < kNumPkFamilies; ++f) {
       if (!p.args[f].words) continue;
-      unsigned &b = p.blocks[f];
+      unsigned &b = p.slots[f];
       if (pass == 0)
-        b = (unsigned)std::min(task_grid(np, per[f], buckets[f]), (int64_t)4 * cus * kPkFamilies[f].waves);
+        b = (unsigned)std::min((task_grid(np, per[f], buckets[f]) + kPkBlockWaves - 1) / kPkBlockWaves * kPkBlockWaves,
+                               (int64_t)4 * cus * kPkFamilies[f].waves);
       else
-        b = (unsigned)(b * ((double)room / (double)full));
+        b = (unsigned)(b * ((double)room / (double)full)) / kPkBlockWaves * kPkBlockWaves;
       if (!b) return 0;  // no room for a slot of every family
       int64_t &r = p.region[family_worker(kFirstPkFamily + f)];
       r = std::max(r, 4 * (int64_t)b * p.args[f].words);
@@ -618,7 +628,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
                          d_pairs, order, plan, out};
   unsigned grid[kNumFamilies];
   for (int f = 0; f < kNumFamilies; ++f) {
-    const int64_t g = f >= kFirstPkFamily ? pk.blocks[f - kFirstPkFamily]
+    const int64_t g = f >= kFirstPkFamily ? pk.slots[f - kFirstPkFamily]
                                           : family_grid(f, np, kb_lo, kb_hi, pk.map);
     if (g > 0x7FFFFFFF)
       return set_err(ctx, CRISPY_ERR_ARG, "%lld pairs need %lld wave tasks in one launch; split the call",
@@ -632,7 +642,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
       (uintptr_t)pk.map.pk_top, (uintptr_t)pk.map.pk_cap, (uintptr_t)nw.dirs.p,
       (uintptr_t)pk.region[0], (uintptr_t)pk.args[0].pack_hi};
   for (unsigned g : grid) key.push_back(g);
-  for (const PkLaunchArgs &k : pk.args) key.push_back((uintptr_t)k.words);
+  for (const PkLaunchArgs &k : pk.args) key.push_back((uintptr_t)k.words * 8 + k.block_waves);
   uint64_t kernels = rs.ext ? 1 : 2;
   for (int f = 0; f < kNumFamilies; ++f) kernels |= grid[f] ? uint64_t(4) << f : 0;
   for (int f = 0; f < kNumPkFamilies; ++f) kernels |= pk.args[f].f16 ? uint64_t(4) << (kNumFamilies + f) : 0;

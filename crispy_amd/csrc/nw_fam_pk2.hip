@@ -4,8 +4,8 @@
 
 namespace crispy {
 
-void launch_nw_pk_family2(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k) {
-  launch_nw_pk_family<2>(s, blocks, a, k);
+void launch_nw_pk_family2(hipStream_t s, unsigned slots, const NwFusedArgs &a, const PkLaunchArgs &k) {
+  launch_nw_pk_family<2>(s, slots, a, k);
 }
 
 }  // namespace crispy

@@ -4,8 +4,8 @@
 
 namespace crispy {
 
-void launch_nw_pk_family3(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k) {
-  launch_nw_pk_family<3>(s, blocks, a, k);
+void launch_nw_pk_family3(hipStream_t s, unsigned slots, const NwFusedArgs &a, const PkLaunchArgs &k) {
+  launch_nw_pk_family<3>(s, slots, a, k);
 }
 
 }  // namespace crispy

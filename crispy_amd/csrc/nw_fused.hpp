@@ -45,6 +45,7 @@ constexpr int kNumPkFamilies = 4;
 constexpr PkFamily kPkFamilies[kNumPkFamilies] = {{1, 16, 5, 4}, {17, 24, 4, 3}, {25, 32, 4, 3}, {33, kPkMaxCells, 3, 2}};
 constexpr int kFirstPkFamily = kNumRegFamilies + kNumSliceWidths;
 constexpr int kNumFamilies = kFirstPkFamily + kNumPkFamilies;
+constexpr int kPkBlockWaves = 4;  // waves (direction slots) per block, at most
 constexpr int kPkTraceSteps = 8;  // steps of directions staged in LDS at a time by the trace
 
 __host__ __device__ constexpr int pk_lanes(int kb, int cap) { return (2 * kb + 1 + 2 * cap - 1) / (2 * cap); }
@@ -128,26 +129,28 @@ struct NwFusedArgs {
   NwPlan *plan;
   float *out;
 };
-// A packed family's launch: one direction slot per block, the slice width cap,
+// A packed family's launch: one direction slot per wave, the slice width cap,
 // and the read set's upper code bits (null when every read is ACGT only).
 struct PkLaunchArgs {
   uint32_t *dirs;
   int64_t words;  // per slot
   int cap;
+  unsigned block_waves;
   bool f16;  // every key of the family's buckets is at most kPkF16Top
   const uint32_t *pack_hi;
 };
 
-// Each launcher runs `blocks` one-wave blocks of its family.
+// Each launcher runs `blocks` one-wave blocks of its family, a packed one
+// `slots` waves in blocks of k.block_waves.
 void launch_nw_reg_family0(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
 void launch_nw_reg_family1(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
 void launch_nw_reg_family2(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
 void launch_nw_reg_family3(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
 void launch_nw_sliced_family24(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
 void launch_nw_sliced_family32(hipStream_t s, unsigned blocks, const NwFusedArgs &a);
-void launch_nw_pk_family0(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k);
-void launch_nw_pk_family1(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k);
-void launch_nw_pk_family2(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k);
-void launch_nw_pk_family3(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k);
+void launch_nw_pk_family0(hipStream_t s, unsigned slots, const NwFusedArgs &a, const PkLaunchArgs &k);
+void launch_nw_pk_family1(hipStream_t s, unsigned slots, const NwFusedArgs &a, const PkLaunchArgs &k);
+void launch_nw_pk_family2(hipStream_t s, unsigned slots, const NwFusedArgs &a, const PkLaunchArgs &k);
+void launch_nw_pk_family3(hipStream_t s, unsigned slots, const NwFusedArgs &a, const PkLaunchArgs &k);
 
 }  // namespace crispy

@@ -495,10 +495,10 @@ __device__ __forceinline__ void nw_pk_wave(const uint32_t *__restrict__ pack, co
   int tb = (tlast - 1) / kPkTraceSteps * kPkTraceSteps;
   fetch(tb);
   for (; tb >= 0; tb -= kPkTraceSteps) {
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the wave's own LDS: its operations are in order
 #pragma unroll
     for (int q = 0; q < NW; ++q) stage[q * 64 + lane] = pre[q];
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     if (tb > 0) fetch(tb - kPkTraceSteps);
     while (__ballot(act && tt > tb)) {
       if (act && tt > tb) {
@@ -565,17 +565,22 @@ __device__ __forceinline__ void pk_dispatch(const int c, const NwFusedArgs &a, c
 
 // Packed kernel for slice widths LO..HI (family F).  The grid is the number
 // of direction slots (about the waves the chip holds), so the scratch is
-// bounded whatever the pair count: a block keeps its slot and takes the
+// bounded whatever the pair count: a wave keeps its slot and takes the
 // family's tasks one after the other, longest first, from a device counter.
+// Blocks of one wave, or of kPkBlockWaves = 4 independent ones (pk_plan in nw.hip).
 template <int LO, int HI, int WAVES, int F, bool EXT, bool F16>
-__global__ __launch_bounds__(64, WAVES) void nw_pk_fused_kernel(const NwFusedArgs a, const PkLaunchArgs x) {
-  __shared__ uint32_t stage[kPkTraceSteps * pk_dir_words(HI) * 64];
-  uint32_t *dirs = x.dirs + (int64_t)blockIdx.x * x.words;
+__global__ __launch_bounds__(64 * kPkBlockWaves, WAVES) void nw_pk_fused_kernel(const NwFusedArgs a, const PkLaunchArgs x) {
+  constexpr int kStage = kPkTraceSteps * pk_dir_words(HI) * 64;
+  extern __shared__ uint32_t stages[];  // kStage words per wave
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const uint32_t slot = blockIdx.x * (blockDim.x >> 6) + (uint32_t)wv;
+  uint32_t *stage = stages + wv * kStage;
+  uint32_t *dirs = x.dirs + (int64_t)slot * x.words;
   NwPlan *plan = a.plan;
   const uint32_t ntasks = plan->ntasks[F];
   const int nbk = (int)plan->nbuckets[F];
   const uint2 *list = plan->list[F];
-  uint32_t t = blockIdx.x;
+  uint32_t t = slot;
   while (t < ntasks) {
     int k = 0;
     for (int base = 0; base < nbk; base += 64) {
@@ -592,19 +597,21 @@ __global__ __launch_bounds__(64, WAVES) void nw_pk_fused_kernel(const NwFusedArg
     pk_dispatch<HI, LO, EXT, F16>(pk_cells(kb, x.cap), a, x, a.order + bk.x, (int32_t)bk.y, kb, G, wave, dirs, stage);
     uint32_t n = 0;
     if ((threadIdx.x & 63) == 0) n = atomicAdd(&plan->next[F], 1u);
-    t = gridDim.x + (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
+    t = gridDim.x * (blockDim.x >> 6) + (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
   }
 }
 
 template <int P>
-inline void launch_nw_pk_family(hipStream_t s, unsigned blocks, const NwFusedArgs &a, const PkLaunchArgs &k) {
+inline void launch_nw_pk_family(hipStream_t s, unsigned slots, const NwFusedArgs &a, const PkLaunchArgs &k) {
   constexpr PkFamily fam = kPkFamilies[P];
+  const unsigned blocks = slots / k.block_waves, threads = 64 * k.block_waves;
+  const size_t lds = sizeof(uint32_t) * kPkTraceSteps * pk_dir_words(fam.hi) * 64 * k.block_waves;
   if (k.pack_hi)
-    nw_pk_fused_kernel<fam.lo, fam.hi, fam.ext_waves, kFirstPkFamily + P, true, false><<<blocks, 64, 0, s>>>(a, k);
+    nw_pk_fused_kernel<fam.lo, fam.hi, fam.ext_waves, kFirstPkFamily + P, true, false><<<blocks, threads, lds, s>>>(a, k);
   else if (k.f16)
-    nw_pk_fused_kernel<fam.lo, fam.hi, fam.waves, kFirstPkFamily + P, false, true><<<blocks, 64, 0, s>>>(a, k);
+    nw_pk_fused_kernel<fam.lo, fam.hi, fam.waves, kFirstPkFamily + P, false, true><<<blocks, threads, lds, s>>>(a, k);
   else
-    nw_pk_fused_kernel<fam.lo, fam.hi, fam.waves, kFirstPkFamily + P, false, false><<<blocks, 64, 0, s>>>(a, k);
+    nw_pk_fused_kernel<fam.lo, fam.hi, fam.waves, kFirstPkFamily + P, false, false><<<blocks, threads, lds, s>>>(a, k);
 }
 
 }  // namespace crispy
