@@ -18,15 +18,31 @@ int set_err(crispy_ctx *ctx, int code, const char *fmt, ...) {
   return code;
 }
 
+// Gives the NW directions' scratch back unless a phase in preparation uses it:
+// it must not keep another buffer from growing.
+static bool drop_scratch(crispy_ctx *ctx) {
+  DevBuf &d = ctx->nw.dirs;
+  if (!d.p || ctx->nw.dirs_busy || hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+  (void)hipFree(d.p);
+  ctx->dev_bytes -= (int64_t)d.bytes;
+  d.p = nullptr;
+  d.bytes = 0;
+  return true;
+}
+
 // Grow-only device buffer.
 int ensure(crispy_ctx *ctx, DevBuf &b, size_t bytes) {
   if (bytes == 0) bytes = 256;
   if (b.bytes >= bytes) return CRISPY_OK;
   // the direction scratch has a limit of its own in a served job
   const bool apart = ctx->scratch_limit >= 0, scratch = &b == &ctx->nw.dirs;
-  const int64_t held = ctx->dev_bytes - (apart && !scratch ? (int64_t)ctx->nw.dirs.bytes : 0);
-  if (apart && scratch ? (int64_t)bytes > ctx->scratch_limit
-                       : ctx->mem_limit > 0 && held - (int64_t)b.bytes + (int64_t)bytes > ctx->mem_limit)
+  int64_t held = 0;
+  auto over = [&]() {
+    held = ctx->dev_bytes - (apart && !scratch ? (int64_t)ctx->nw.dirs.bytes : 0);
+    return apart && scratch ? (int64_t)bytes > ctx->scratch_limit
+                            : ctx->mem_limit > 0 && held - (int64_t)b.bytes + (int64_t)bytes > ctx->mem_limit;
+  };
+  if (over() && (scratch || apart || !drop_scratch(ctx) || over()))
     return set_err(ctx, CRISPY_ERR_NOMEM, "growing a buffer to %zu bytes would take the context past its "
                    "device memory limit (%lld of %lld bytes held)", bytes, (long long)held,
                    (long long)ctx->mem_limit);
@@ -38,6 +54,10 @@ int ensure(crispy_ctx *ctx, DevBuf &b, size_t bytes) {
     b.bytes = 0;
   }
   hipError_t e = hipMalloc(&b.p, bytes);
+  if (e != hipSuccess && !scratch && drop_scratch(ctx)) {
+    (void)hipGetLastError();
+    e = hipMalloc(&b.p, bytes);
+  }
   if (e != hipSuccess) {
     b.p = nullptr;
     (void)hipGetLastError();

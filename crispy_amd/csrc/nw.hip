@@ -581,11 +581,15 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   // Pairs of reads with other bytes run packed up to ext_top; what the fused
   // kernels cannot take exists only if the reads allow it.
   const int64_t generic_bytes = (std::min<int64_t>(np, 32768) + 255) / 256 * 256 * sizeof(int2) * (rs.maxlen + 1);
-  const int64_t later = 24 * (np + 1) + (1 << 20) + (rs.all_clean ? 0 : generic_bytes);  // the filter's buffers
+  const int64_t later = 40 * (np + 1) + (4 << 20) + (rs.all_clean ? 0 : generic_bytes);  // the sort and the filter
   const int64_t room = ctx->scratch_limit >= 0 ? ctx->scratch_limit
                        : ctx->mem_limit > 0    ? ctx->mem_limit - ctx->dev_bytes + (int64_t)nw.dirs.bytes - later
                                                : kPkScratchBytes;
   PkPlan pk = pk_plan(ctx->cus, np, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, room);
+  struct Busy {
+    NwState &nw;
+    ~Busy() { nw.dirs_busy = false; }
+  } busy{nw};
   if (pk.bytes() > 0) {
     const int rc = ensure(ctx, nw.dirs, (size_t)pk.bytes());
     if (rc == CRISPY_ERR_NOMEM) {  // a device that others fill: the unpacked kernels need no scratch
@@ -595,6 +599,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
       return rc;
     }
   }
+  nw.dirs_busy = true;
   for (int f = 0; f < kNumPkFamilies; ++f) {
     static_assert(kNumWorkers == 2, "the second worker's region follows the first's");
     pk.args[f].dirs = nw.dirs.as<uint32_t>() + (family_worker(kFirstPkFamily + f) ? pk.region[0] / 4 : 0);

@@ -77,3 +77,35 @@ def test_packed_equals_unpacked_and_oracle(name):
             assert limit < 0 or held <= limit
             if limit < 0:
                 assert held > 0 or len(other) > 12
+
+
+def test_scratch_makes_room_for_other_buffers():
+    """Under a memory limit that holds a job without directions' scratch, a
+    smaller job's scratch is given back when the larger one's buffers grow."""
+    print("scratch makes room", flush=True)
+    rng = np.random.default_rng(5)
+    small = ca.Reads.from_list(_reads(rng, 300, 200, 300, b""))
+    large = ca.Reads.from_list(_reads(rng, 6000, 200, 300, b""))
+    pairs = rng.integers(0, 300, (40000, 2)).astype(np.int32)
+
+    def job(ctx, reads):
+        ctx.upload_reads(ca.KMER, reads)
+        ctx.upload_reads(ca.NW, reads)
+        ctx.kmer_run(6, 0.3)
+        return ctx.nw_dists(pairs, 10)
+
+    with ca.Context(0) as ctx:
+        lib = ctx._L
+        lib.crispy_ctx_scratch_bytes.restype = ctypes.c_int64
+        ctx._check(lib.crispy_ctx_set_scratch_limit(ctx._h, ctypes.c_int64(0)))
+        want = [job(ctx, small), job(ctx, large)]
+        need = ctx.device_bytes()
+    with ca.Context(0) as ctx:
+        ctx._check(lib.crispy_ctx_set_mem_limit(ctx._h, ctypes.c_int64(need + (1 << 20))))
+        got = job(ctx, small)
+        assert np.array_equal(got, want[0])
+        assert lib.crispy_ctx_scratch_bytes(ctx._h) > 0
+        for _ in range(2):
+            got = job(ctx, large)
+            assert np.array_equal(got, want[1])
+            assert ctx.device_bytes() <= need + (1 << 20)
