@@ -36,7 +36,6 @@ constexpr int kGenericBucket = kKbSliceMax + 1;
 // k-mer tile geometry.
 constexpr int kTile = 128;        // reads per tile side
 constexpr int kChunkWords = 16;   // bitmap words staged in LDS per step of the tile kernel
-constexpr int kBitmapSlack = 32;  // words after the last bitmap row: a last chunk may be staged whole
 // Buckets of the hashed k = 6 candidate filter: 1,280, 1,536 or 2,048 (40,
 // 48 or 64 bitmap words per read, in 8-word groups); fewer buckets mean less
 // tile work and more candidates for the exact passes.

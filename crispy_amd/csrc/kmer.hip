@@ -954,7 +954,8 @@ __global__ __launch_bounds__(256, 2) void kmer_sweep_kernel(
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const lds_f4 v = *reinterpret_cast<const lds_f4 *>(&sG[wv][fa * 32 + 4 * g + 8 * q]);
-      gq[fa][q] = min(min(__float_as_uint(v[0]), __float_as_uint(v[1])), min(__float_as_uint(v[2]), __float_as_uint(v[3])));
+      gq[fa][q] = min(min(__float_as_uint(v[0]), __float_as_uint(v[1])),
+                      min(__float_as_uint(v[2]), __float_as_uint(v[3])));
     }
     grmin[fa] = min(min(gq[fa][0], gq[fa][1]), min(gq[fa][2], gq[fa][3]));
   }
@@ -1105,7 +1106,8 @@ __global__ __launch_bounds__(256, 2) void kmer_sweep_kernel(
             const uint32_t id = (uint32_t)((fa * 8 + 2 * q + g) << 11) | (uint32_t)(c * kTile + fb * 32 + r32);
             queue[qcount + (int)below] =
                 make_uint2((uint32_t)acc[fa][fb][4 * q] | (uint32_t)acc[fa][fb][4 * q + 1] << 11 | id << 22,
-                           (uint32_t)acc[fa][fb][4 * q + 2] | (uint32_t)acc[fa][fb][4 * q + 3] << 11 | (id >> 10) << 22);
+                           (uint32_t)acc[fa][fb][4 * q + 2] | (uint32_t)acc[fa][fb][4 * q + 3] << 11 |
+                               (id >> 10) << 22);
           }
           qcount += __popcll(ball);
         });

@@ -42,7 +42,8 @@ struct PkFamily {
   int ext_waves;  // with the upper code bits
 };
 constexpr int kNumPkFamilies = 4;
-constexpr PkFamily kPkFamilies[kNumPkFamilies] = {{1, 16, 5, 4}, {17, 24, 4, 3}, {25, 32, 4, 3}, {33, kPkMaxCells, 3, 2}};
+constexpr PkFamily kPkFamilies[kNumPkFamilies] = {
+    {1, 16, 5, 4}, {17, 24, 4, 3}, {25, 32, 4, 3}, {33, kPkMaxCells, 3, 2}};
 constexpr int kFirstPkFamily = kNumRegFamilies + kNumSliceWidths;
 constexpr int kNumFamilies = kFirstPkFamily + kNumPkFamilies;
 constexpr int kPkBlockWaves = 4;  // waves (direction slots) per block, at most

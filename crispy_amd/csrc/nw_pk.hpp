@@ -569,7 +569,8 @@ __device__ __forceinline__ void pk_dispatch(const int c, const NwFusedArgs &a, c
 // family's tasks one after the other, longest first, from a device counter.
 // Blocks of one wave, or of kPkBlockWaves = 4 independent ones (pk_plan in nw.hip).
 template <int LO, int HI, int WAVES, int F, bool EXT, bool F16>
-__global__ __launch_bounds__(64 * kPkBlockWaves, WAVES) void nw_pk_fused_kernel(const NwFusedArgs a, const PkLaunchArgs x) {
+__global__ __launch_bounds__(64 * kPkBlockWaves, WAVES) void nw_pk_fused_kernel(const NwFusedArgs a,
+                                                                                const PkLaunchArgs x) {
   constexpr int kStage = kPkTraceSteps * pk_dir_words(HI) * 64;
   extern __shared__ uint32_t stages[];  // kStage words per wave
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -607,7 +608,8 @@ inline void launch_nw_pk_family(hipStream_t s, unsigned slots, const NwFusedArgs
   const unsigned blocks = slots / k.block_waves, threads = 64 * k.block_waves;
   const size_t lds = sizeof(uint32_t) * kPkTraceSteps * pk_dir_words(fam.hi) * 64 * k.block_waves;
   if (k.pack_hi)
-    nw_pk_fused_kernel<fam.lo, fam.hi, fam.ext_waves, kFirstPkFamily + P, true, false><<<blocks, threads, lds, s>>>(a, k);
+    nw_pk_fused_kernel<fam.lo, fam.hi, fam.ext_waves, kFirstPkFamily + P, true, false>
+        <<<blocks, threads, lds, s>>>(a, k);
   else if (k.f16)
     nw_pk_fused_kernel<fam.lo, fam.hi, fam.waves, kFirstPkFamily + P, false, true><<<blocks, threads, lds, s>>>(a, k);
   else

@@ -291,7 +291,8 @@ int64_t crispy_server_job_bytes(const char *bases, const int64_t *offsets, int32
   int64_t prof = (int64_t)n * (4 * words_per_read(K) + 48) + 6 * nbases;
   // K > 6, and large K = 6 jobs: K-mer lists, the hashed k = 6 bitmaps (at most
   // 2,048 bits) and their excess and bounds, candidates + their refined copy, the 256 x 4 KB segment counters
-  if (K > 6 || (K == 6 && all_pairs >= kCandidatePairs)) prof += 2 * nbases + 16 * (int64_t)n + 260 * (int64_t)n + 16 * (std::max(guess, pairs) + 256) + (1 << 20);
+  if (K > 6 || (K == 6 && all_pairs >= kCandidatePairs))
+    prof += 2 * nbases + 16 * (int64_t)n + 260 * (int64_t)n + 16 * (std::max(guess, pairs) + 256) + (1 << 20);
   int64_t est = reads + prof + 12 * guess + 72 * pairs + (int64_t)(8 << 20);
   const bool generic = band <= 1 || !clean || (band > 0 && maxlen / band > kSlicedMaxHalfBand);
   if (generic) est += 8 * std::min<int64_t>(pairs, 32768) * (maxlen + 1);
