@@ -578,10 +578,20 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   float *out = nw.dist.as<float>();
   NwPlan *plan = nw.plan.as<NwPlan>();
 
+  // The sort's temporary storage first: what the call cannot do without must
+  // not find the memory taken by the directions' scratch.
+  const BucketKey bkey = bucket_key(kb_lo, std::min(kb_hi, kKbSliceMax), rs.maxlen);
+  size_t tbytes = 0;
+  CRISPY_HIP(ctx, rocprim::radix_sort_pairs<RadixOnesweep>(nullptr, tbytes, nw.keys.as<uint32_t>(),
+                                            nw.keys_alt.as<uint32_t>(), nw.idx.as<uint32_t>(), order,
+                                            (size_t)np, 0, bkey.bits, ctx->stream));
+  CRISPY_TRY(ensure(ctx, ctx->temp, tbytes));
+
   // Pairs of reads with other bytes run packed up to ext_top; what the fused
   // kernels cannot take exists only if the reads allow it.
   const int64_t generic_bytes = (std::min<int64_t>(np, 32768) + 255) / 256 * 256 * sizeof(int2) * (rs.maxlen + 1);
-  const int64_t later = 40 * (np + 1) + (4 << 20) + (rs.all_clean ? 0 : generic_bytes);  // the sort and the filter
+  const bool some_generic = kb_hi > kKbSliceMax || !rs.all_clean;
+  const int64_t later = 24 * (np + 1) + (4 << 20) + (some_generic ? generic_bytes : 0);  // the filter, the generic kernel
   const int64_t room = ctx->scratch_limit >= 0 ? ctx->scratch_limit
                        : ctx->mem_limit > 0    ? ctx->mem_limit - ctx->dev_bytes + (int64_t)nw.dirs.bytes - later
                                                : kPkScratchBytes;
@@ -610,7 +620,6 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
 
   // bucketing: launched one by one (the radix sort clears its own state
   // with memsets, which stay out of graphs)
-  const BucketKey bkey = bucket_key(kb_lo, std::min(kb_hi, kKbSliceMax), rs.maxlen);
   hipEvent_t ev;
   CRISPY_HIP(ctx, hipMemsetAsync(nw.hist.p, 0, sizeof(unsigned int) * kNumBuckets, ctx->stream));
   CRISPY_HIP(ctx, hipMemsetAsync(nw.cells.p, 0, sizeof(unsigned long long) * kNumBuckets, ctx->stream));
@@ -619,11 +628,6 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
       d_pairs, np, rs.len.as<int32_t>(), rs.clean.as<uint8_t>(), band, ext_top, bkey, nw.keys.as<uint32_t>(),
       nw.idx.as<uint32_t>(), nw.hist.as<unsigned int>(), nw.cells.as<unsigned long long>());
   CRISPY_LAUNCHED(ctx);
-  size_t tbytes = 0;
-  CRISPY_HIP(ctx, rocprim::radix_sort_pairs<RadixOnesweep>(nullptr, tbytes, nw.keys.as<uint32_t>(),
-                                            nw.keys_alt.as<uint32_t>(), nw.idx.as<uint32_t>(), order,
-                                            (size_t)np, 0, bkey.bits, ctx->stream));
-  CRISPY_TRY(ensure(ctx, ctx->temp, tbytes));
   CRISPY_HIP(ctx, rocprim::radix_sort_pairs<RadixOnesweep>(ctx->temp.p, tbytes, nw.keys.as<uint32_t>(),
                                             nw.keys_alt.as<uint32_t>(), nw.idx.as<uint32_t>(), order,
                                             (size_t)np, 0, bkey.bits, ctx->stream));
@@ -671,6 +675,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
     CRISPY_HIP(ctx, hipMemcpyAsync(h_g, &plan->btab[kGenericBucket], sizeof(uint2), hipMemcpyDeviceToHost,
                                    ctx->stream));
     CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    nw.dirs_busy = false;  // the families are done
     const uint2 gb = *h_g;
     const int64_t ng = gb.y;
     if (ng > 0) {
