@@ -18,15 +18,21 @@ int set_err(crispy_ctx *ctx, int code, const char *fmt, ...) {
   return code;
 }
 
-// Gives the NW directions' scratch back unless a phase in preparation uses it:
-// it must not keep another buffer from growing.
-static bool drop_scratch(crispy_ctx *ctx) {
-  DevBuf &d = ctx->nw.dirs;
-  if (!d.p || ctx->nw.dirs_busy || hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
-  (void)hipFree(d.p);
-  ctx->dev_bytes -= (int64_t)d.bytes;
-  d.p = nullptr;
-  d.bytes = 0;
+// Frees what the context can do without, so that it never keeps buffer b from
+// growing: the NW directions' scratch (if `dirs`) and the upper code bits of
+// reads with other bytes, whose pairs then take the slower kernels.  Not while
+// an NW phase in preparation uses them.  True if something was freed.
+static bool make_room(crispy_ctx *ctx, const DevBuf &b, bool dirs) {
+  ReadStore &rs = ctx->reads[CRISPY_READS_NW];
+  dirs = dirs && ctx->nw.dirs.p;
+  const bool hi = &b != &rs.pack_hi && rs.pack_hi.p;
+  if (&b == &ctx->nw.dirs || ctx->nw.busy || !(dirs || hi)) return false;
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+  if (dirs) release(ctx, ctx->nw.dirs);
+  if (hi) {
+    release(ctx, rs.pack_hi);
+    rs.ext = false;
+  }
   return true;
 }
 
@@ -42,7 +48,7 @@ int ensure(crispy_ctx *ctx, DevBuf &b, size_t bytes) {
     return apart && scratch ? (int64_t)bytes > ctx->scratch_limit
                             : ctx->mem_limit > 0 && held - (int64_t)b.bytes + (int64_t)bytes > ctx->mem_limit;
   };
-  if (over() && (scratch || apart || !drop_scratch(ctx) || over()))
+  if (over() && (!make_room(ctx, b, !apart) || over()))
     return set_err(ctx, CRISPY_ERR_NOMEM, "growing a buffer to %zu bytes would take the context past its "
                    "device memory limit (%lld of %lld bytes held)", bytes, (long long)held,
                    (long long)ctx->mem_limit);
@@ -54,7 +60,7 @@ int ensure(crispy_ctx *ctx, DevBuf &b, size_t bytes) {
     b.bytes = 0;
   }
   hipError_t e = hipMalloc(&b.p, bytes);
-  if (e != hipSuccess && !scratch && drop_scratch(ctx)) {
+  if (e != hipSuccess && make_room(ctx, b, true)) {
     (void)hipGetLastError();
     e = hipMalloc(&b.p, bytes);
   }
@@ -392,9 +398,8 @@ int crispy_reads_upload(crispy_ctx *ctx, int slot, const char *bases, const int6
   if (n < 0 || n > CRISPY_MAX_NUM_READS || (n > 0 && (!bases || !offsets)))
     return set_err(ctx, CRISPY_ERR_ARG, "unsupported numReads: %d", n);
   CRISPY_HIP(ctx, hipSetDevice(ctx->device));
-  ReadStore &rs = ctx->reads[slot];
-  rs.n = n;
-  rs.h_len.assign(n, 0);
+  // A call refused for its arguments leaves the slot as it was.
+  std::vector<int32_t> lens(n, 0);
   std::vector<int64_t> poff(n + 1, 0);
   int32_t maxlen = 0, minlen = CRISPY_MAX_READ_LEN;
   if (n > 0 && offsets[0] != 0) return set_err(ctx, CRISPY_ERR_ARG, "offsets[0] must be 0");
@@ -402,14 +407,19 @@ int crispy_reads_upload(crispy_ctx *ctx, int slot, const char *bases, const int6
     const int64_t L = offsets[r + 1] - offsets[r];
     if (L < 1 || L > CRISPY_MAX_READ_LEN)
       return set_err(ctx, CRISPY_ERR_ARG, "unsupported read length %lld (read %d)", (long long)L, r);
-    rs.h_len[r] = (int32_t)L;
+    lens[r] = (int32_t)L;
     maxlen = std::max<int32_t>(maxlen, (int32_t)L);
     minlen = std::min<int32_t>(minlen, (int32_t)L);
     poff[r + 1] = poff[r] + (L + 15) / 16 + 1;  // one zero pad word per read
   }
+  // One that fails from here on leaves it empty: its buffers may be short or
+  // gone, so no later call may find reads in it.
+  ReadStore &rs = ctx->reads[slot];
+  rs.n = 0;
+  rs.maxlen = rs.minlen = 0;
+  rs.ext = false;
   rs.nbases = n ? offsets[n] : 0;
-  rs.maxlen = maxlen;
-  rs.minlen = n ? minlen : 0;
+  rs.h_len = std::move(lens);
   const int64_t nwords = poff[n];
   CRISPY_TRY(ensure(ctx, rs.bases, (size_t)rs.nbases + 16));
   CRISPY_TRY(ensure(ctx, rs.off, sizeof(int64_t) * (n + 1)));
@@ -418,7 +428,7 @@ int crispy_reads_upload(crispy_ctx *ctx, int slot, const char *bases, const int6
   CRISPY_TRY(ensure(ctx, rs.pack, sizeof(uint32_t) * (nwords + 4)));
   CRISPY_TRY(ensure(ctx, rs.clean, (size_t)n + 1));
   CRISPY_TRY(ensure(ctx, rs.other, 256 / 8));
-  rs.ext = false;
+  bool ext = false;
   if (n > 0) {
     uint32_t other[8] = {};
     CRISPY_HIP(ctx, hipMemcpyAsync(rs.bases.p, bases, rs.nbases, hipMemcpyHostToDevice, ctx->stream));
@@ -447,9 +457,17 @@ int crispy_reads_upload(crispy_ctx *ctx, int slot, const char *bases, const int6
         if (distinct < 12) codes.code[c] = (uint8_t)(4 + distinct);
         ++distinct;
       }
-    rs.ext = slot == CRISPY_READS_NW && distinct > 0 && distinct <= 12;
-    if (rs.ext) {
-      CRISPY_TRY(ensure(ctx, rs.pack_hi, sizeof(uint32_t) * (nwords + 4)));
+    ext = slot == CRISPY_READS_NW && distinct > 0 && distinct <= 12;
+    if (ext) {
+      const int rc = ensure(ctx, rs.pack_hi, sizeof(uint32_t) * (nwords + 4));
+      if (rc == CRISPY_ERR_NOMEM) {  // the generic kernel takes those pairs, from the bytes
+        ctx->err.clear();
+        ext = false;
+      } else if (rc != CRISPY_OK) {
+        return rc;
+      }
+    }
+    if (ext) {
       pack_ext_kernel<<<n, 256, 0, ctx->stream>>>(rs.bases.as<uint8_t>(), rs.off.as<int64_t>(), rs.poff.as<int64_t>(),
                                                   rs.clean.as<uint8_t>(), codes, rs.pack.as<uint32_t>(),
                                                   rs.pack_hi.as<uint32_t>());
@@ -458,6 +476,10 @@ int crispy_reads_upload(crispy_ctx *ctx, int slot, const char *bases, const int6
   }
   rs.all_clean = 1;
   for (int32_t r = 0; r < n; ++r) rs.all_clean &= rs.h_clean[r];
+  rs.maxlen = maxlen;
+  rs.minlen = n ? minlen : 0;
+  rs.ext = ext;
+  rs.n = n;
   rs.generation += 1;
   if (slot == CRISPY_READS_KMER) ctx->km.valid = false;
   ctx->nw.valid = false;

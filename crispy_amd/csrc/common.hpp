@@ -146,6 +146,7 @@ struct KmerState {
   DevBuf keys, keys_alt, dists, dists_alt, pairs, counter;
   int64_t cap = 0;
   int64_t count = 0;
+  int32_t reads = 0;  // the read count that the result's pairs lie in
   bool valid = false;
   GraphSegment g_profile, g_tile;  // captured profile pass and tile pass
 };
@@ -156,7 +157,7 @@ struct NwState {
   DevBuf plan;  // NwPlan of the DP phase (bucket table, family task lists, counters)
   DevBuf stat;  // cells per family (generic last) summed over timed runs
   DevBuf dirs;  // direction slots of the packed families
-  bool dirs_busy = false;  // a phase in preparation points into them: not given back to make room
+  bool busy = false;  // a phase in preparation uses dirs and the reads' pack_hi: not freed to make room
   DevBuf csr_rows, csr_cols;  // CSR view of the (i, j)-ordered result
   DevBuf sort_k0, sort_k1, sort_b0, sort_b1, sort_pairs, sort_dists;  // (dist, i, j) sorts
   int slice_width = 0;  // sliced-kernel cells per lane: 0 = cost model, 24 or 32 = forced

@@ -1996,6 +1996,7 @@ int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
                    (long long)tile_end);
   const int64_t nt = tile_end - tile_begin;
   km.count = 0;
+  km.reads = n;
   if (n < 2 || nt == 0) {
     km.valid = true;
     if (count) *count = 0;

@@ -598,7 +598,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   PkPlan pk = pk_plan(ctx->cus, np, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, room);
   struct Busy {
     NwState &nw;
-    ~Busy() { nw.dirs_busy = false; }
+    ~Busy() { nw.busy = false; }
   } busy{nw};
   if (pk.bytes() > 0) {
     const int rc = ensure(ctx, nw.dirs, (size_t)pk.bytes());
@@ -609,7 +609,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
       return rc;
     }
   }
-  nw.dirs_busy = true;
+  nw.busy = true;
   for (int f = 0; f < kNumPkFamilies; ++f) {
     static_assert(kNumWorkers == 2, "the second worker's region follows the first's");
     pk.args[f].dirs = nw.dirs.as<uint32_t>() + (family_worker(kFirstPkFamily + f) ? pk.region[0] / 4 : 0);
@@ -675,7 +675,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
     CRISPY_HIP(ctx, hipMemcpyAsync(h_g, &plan->btab[kGenericBucket], sizeof(uint2), hipMemcpyDeviceToHost,
                                    ctx->stream));
     CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    nw.dirs_busy = false;  // the families are done
+    nw.busy = false;  // the families are done
     const uint2 gb = *h_g;
     const int64_t ng = gb.y;
     if (ng > 0) {
@@ -917,7 +917,7 @@ int crispy_nw_run(crispy_ctx *ctx, const int32_t *pairs, int64_t npairs, int ban
 int crispy_nw_run_on_kmer(crispy_ctx *ctx, int band, float threshold, int64_t *count) {
   if (!ctx) return CRISPY_ERR_ARG;
   if (!ctx->km.valid) return set_err(ctx, CRISPY_ERR_STATE, "no k-mer result to consume");
-  if (ctx->reads[CRISPY_READS_NW].n != ctx->reads[CRISPY_READS_KMER].n)
+  if (ctx->reads[CRISPY_READS_NW].n != ctx->km.reads)
     return set_err(ctx, CRISPY_ERR_STATE, "NW read slot does not hold the k-mer reads");
   CRISPY_HIP(ctx, hipSetDevice(ctx->device));
   ctx->nw.valid = false;
@@ -1011,7 +1011,7 @@ int crispy_nw_fetch_sorted(crispy_ctx *ctx, int64_t first, int64_t count, int32_
 int crispy_nw_autotune(crispy_ctx *ctx, int band, int repeats, int *chosen) {
   if (!ctx || repeats < 1) return CRISPY_ERR_ARG;
   if (!ctx->km.valid) return set_err(ctx, CRISPY_ERR_STATE, "no k-mer result to tune on");
-  if (ctx->reads[CRISPY_READS_NW].n != ctx->reads[CRISPY_READS_KMER].n)
+  if (ctx->reads[CRISPY_READS_NW].n != ctx->km.reads)
     return set_err(ctx, CRISPY_ERR_STATE, "NW read slot does not hold the k-mer reads");
   CRISPY_HIP(ctx, hipSetDevice(ctx->device));
   NwState &nw = ctx->nw;

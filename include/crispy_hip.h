@@ -111,7 +111,8 @@ int64_t crispy_band_cells(int32_t len1, int32_t len2, int32_t band);
  * when every byte is one of 'A','C','G','T'.  Replaces the tupleSet /
  * texture upload (kmerCUDA.cu:35-72) and convertToBinary + texture upload
  * (genMain.cpp:280-321, genCUDA.cu:94-144).  Reads stay resident until the
- * slot is re-uploaded or the context is destroyed. */
+ * slot is re-uploaded or the context is destroyed.  A call refused for its
+ * arguments leaves the slot as it was, one that fails later leaves it empty. */
 int crispy_reads_upload(crispy_ctx *ctx, int slot, const char *bases, const int64_t *offsets,
                         int32_t n);
 
