@@ -1975,9 +1975,9 @@ int crispy_kmer_autotune(crispy_ctx *ctx, int K, float threshold, int repeats, i
   return CRISPY_OK;
 }
 
-int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin, int64_t tile_end,
-                    int64_t *count) {
-  if (!ctx) return CRISPY_ERR_ARG;
+// crispy_kmer_run; `in_tile`: K <= 6 counts in the tile whatever the pair count.
+static int kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin, int64_t tile_end, int64_t *count,
+                    bool in_tile) {
   if (K < 1 || K > 8) return set_err(ctx, CRISPY_ERR_ARG, "unsupported K=%d (1..8)", K);
   CRISPY_HIP(ctx, hipSetDevice(ctx->device));
   ReadStore &rs = ctx->reads[CRISPY_READS_KMER];
@@ -2014,8 +2014,13 @@ int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
   // latency-bound merges cost more than the sweep saves.  K < 6 runs its
   // candidate tiles on the exact bitmaps, which win from ~10^9 pairs up.
   // exact_pass 2: the candidate form on the exact bitmaps (no hashing).
-  const bool separate = km.exact_pass >= 1 || (km.exact_pass == -1 &&
+  const bool separate = km.exact_pass >= 1 || (km.exact_pass == -1 && !in_tile &&
                          (int64_t)n * (n - 1) / 2 >= (K == 6 ? kExactPassPairs6 : kExactPassPairs));
+  struct Busy {
+    KmerState &km;
+    ~Busy() { km.busy = false; }
+  } busy{km};
+  km.busy = K > 6 || separate;
   CRISPY_TRY(build_profiles(ctx, KP, K, (K > 6 || separate) && km.exact_pass != 2));
   // the k = 6 candidate tiles: on the hashed bitmaps, or on the exact ones
   const TileFn tiles6 = !km.hashed                          ? launch_tiles<6, true>
@@ -2120,6 +2125,7 @@ int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
       return CRISPY_OK;
     }));
   }
+  km.busy = false;
   CRISPY_TRY(ensure(ctx, km.keys_alt, sizeof(uint64_t) * (km.count + 1)));
   CRISPY_TRY(ensure(ctx, km.dists_alt, sizeof(float) * (km.count + 1)));
   CRISPY_TRY(ensure(ctx, km.pairs, sizeof(int2) * (km.count + 1)));
@@ -2134,6 +2140,20 @@ int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
   km.valid = true;
   if (count) *count = km.count;
   return CRISPY_OK;
+}
+
+int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin, int64_t tile_end,
+                    int64_t *count) {
+  if (!ctx) return CRISPY_ERR_ARG;
+  const int rc = kmer_run(ctx, K, threshold, tile_begin, tile_end, count, false);
+  const int64_t n = ctx->reads[CRISPY_READS_KMER].n, pairs = n * (n - 1) / 2;
+  // No room for the candidates: counts in the tile need none (from
+  // kExactPassPairs up they would take several times as long).
+  if (rc != CRISPY_ERR_NOMEM || K != 6 || ctx->km.exact_pass != -1 || pairs < kExactPassPairs6 ||
+      pairs >= kExactPassPairs)
+    return rc;
+  ctx->err.clear();
+  return kmer_run(ctx, K, threshold, tile_begin, tile_end, count, true);
 }
 
 int crispy_kmer_fetch(crispy_ctx *ctx, int64_t first, int64_t count, int32_t *pairs, float *dists) {

@@ -250,8 +250,23 @@ void worker_loop(crispy_server *srv, int slot) {
 // Widest half band kB = (L1 + L2) / (2 band) the register and sliced NW
 // kernels take (64 lanes x 24 cells per pair); wider pairs use the generic one.
 constexpr int64_t kSlicedMaxHalfBand = (64 * 24 - 1) / 2;
-// K = 6 jobs of this many pairs take hashed candidates (kExactPassPairs6 in kmer.hip).
+// K = 6 jobs of this many pairs take hashed candidates if there is room
+// (kExactPassPairs6 in kmer.hip).
 constexpr int64_t kCandidatePairs = 400000000;
+
+// First size of the k-mer result: the pairs in the tiles, at most 4 Mi.
+int64_t result_guess(int32_t n) {
+  const int64_t nb = (n + 127) / 128;
+  const int64_t tiles = nb * (nb + 1) / 2;
+  return std::min<int64_t>(int64_t(1) << 22, std::max<int64_t>(4096, tiles * 128 * 128));
+}
+
+// The hashed k = 6 bitmaps (at most 2,048 bits) with their excess and bounds,
+// the candidates and their refined copy, the 256 x 4 KB segment counters.
+int64_t candidate_bytes(int32_t n) {
+  const int64_t pairs = std::min<int64_t>((int64_t)n * (n - 1) / 2, 256 * (int64_t)n);
+  return 260 * (int64_t)n + 16 * (std::max(result_guess(n), pairs) + 256) + (1 << 20);
+}
 
 int64_t words_per_read(int K) {
   const int KP = K <= 6 ? K : 6;
@@ -282,17 +297,13 @@ int64_t crispy_server_job_bytes(const char *bases, const int64_t *offsets, int32
     const char c = bases[q];
     clean = c == 'A' || c == 'C' || c == 'G' || c == 'T';
   }
-  const int64_t nb = (n + 127) / 128;
-  const int64_t tiles = nb * (nb + 1) / 2;
-  const int64_t guess = std::min<int64_t>(int64_t(1) << 22, std::max<int64_t>(4096, tiles * 128 * 128));
+  const int64_t guess = result_guess(n);
   const int64_t all_pairs = (int64_t)n * (n - 1) / 2;
   const int64_t pairs = std::min<int64_t>(all_pairs, 256 * (int64_t)n);
   const int64_t reads = 2 * (nbases + nbases / 4 + 48 * (int64_t)n);
   int64_t prof = (int64_t)n * (4 * words_per_read(K) + 48) + 6 * nbases;
-  // K > 6, and large K = 6 jobs: K-mer lists, the hashed k = 6 bitmaps (at most
-  // 2,048 bits) and their excess and bounds, candidates + their refined copy, the 256 x 4 KB segment counters
-  if (K > 6 || (K == 6 && all_pairs >= kCandidatePairs))
-    prof += 2 * nbases + 16 * (int64_t)n + 260 * (int64_t)n + 16 * (std::max(guess, pairs) + 256) + (1 << 20);
+  // K > 6: K-mer lists and the candidates
+  if (K > 6) prof += 2 * nbases + 16 * (int64_t)n + candidate_bytes(n);
   int64_t est = reads + prof + 12 * guess + 72 * pairs + (int64_t)(8 << 20);
   const bool generic = band <= 1 || !clean || (band > 0 && maxlen / band > kSlicedMaxHalfBand);
   if (generic) est += 8 * std::min<int64_t>(pairs, 32768) * (maxlen + 1);
@@ -369,9 +380,13 @@ int64_t crispy_server_submit(crispy_server *srv, const char *kmer_bases, const i
   for (int32_t r = 0; r < n; ++r) lens.push_back(noff[r + 1] - noff[r]);
   std::lock_guard<std::mutex> lk(srv->mu);
   if (job->est > srv->budget) return CRISPY_ERR_NOMEM;  // would never be admitted
-  // What is left of an even share of the budget goes to the directions, so the
-  // slots still run side by side; 2 bits per band position and row.
+  // What is left of an even share of the budget goes to what makes the job
+  // faster, so the slots still run side by side: a large K = 6 job's candidates,
+  // then the directions, 2 bits per band position and row.
   {
+    if (K == 6 && (int64_t)n * (n - 1) / 2 >= kCandidatePairs &&
+        job->est + candidate_bytes(n) <= srv->budget / (int64_t)srv->ctxs.size())
+      job->est += candidate_bytes(n);
     const int64_t len = n > 0 ? *std::max_element(lens.begin(), lens.end()) : 0;
     const int64_t kb = band >= 2 ? len / band : len;
     const double want = 1.5 * std::min<double>((double)n * (n - 1) / 2, 256.0 * n) * (len + 32) * (2 * kb + 32) / 4;
