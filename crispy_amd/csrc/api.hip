@@ -136,6 +136,12 @@ void timer_end(crispy_ctx *ctx, const char *name, hipEvent_t a, double units, hi
   ctx->pending.push_back(PendingEvent{name, a, b, units});
 }
 
+int wait_main(crispy_ctx *ctx) {
+  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->settled = ctx->launches;
+  return CRISPY_OK;
+}
+
 // Work queued on `stream` so far happens before anything later queued on the
 // workers.
 int fork_workers(crispy_ctx *ctx) {
@@ -382,8 +388,7 @@ int crispy_host_free(void *ptr) {
 
 int crispy_ctx_sync(crispy_ctx *ctx) {
   if (!ctx) return CRISPY_ERR_ARG;
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return CRISPY_OK;
+  return wait_main(ctx);
 }
 
 int64_t crispy_ctx_device_bytes(const crispy_ctx *ctx) { return ctx ? ctx->dev_bytes : 0; }

@@ -112,11 +112,14 @@ struct ReadStore {
   int generation = 0;  // bumped on every upload (invalidates cached profiles)
 };
 
-// A captured graph of a launch sequence and the arguments it was captured
-// with (pointers, sizes, scalars); captured again when they change.
+// The instantiated graph of a launch sequence (graph_segment.hpp): the
+// arguments (pointers, sizes, scalars) and kernels it was captured with, the
+// arguments of the last run without it, and its last launch (crispy_ctx::launches).
 struct GraphSegment {
   hipGraphExec_t exec = nullptr;
-  std::vector<uintptr_t> key;
+  std::vector<uintptr_t> key, seen;
+  std::vector<const void *> kernels;
+  uint64_t launch = 0;
 };
 
 struct KmerState {
@@ -163,15 +166,12 @@ struct NwState {
   DevBuf sort_k0, sort_k1, sort_b0, sort_b1, sort_pairs, sort_dists;  // (dist, i, j) sorts
   int slice_width = 0;  // sliced-kernel cells per lane: 0 = cost model, 24 or 32 = forced
   // Captured DP phases, one per set of kernels (the kernel families that a
-  // job's read lengths and pair count put to work), and the filter.  A job of
-  // another set takes another graph: an instantiated graph is only ever
-  // updated with new arguments of the same kernels, and a server's slots,
-  // whose jobs alternate between a few sets, do not destroy and instantiate
-  // graphs job after job.
+  // run's read lengths and pair count put to work), so that runs which
+  // alternate between a few sets keep their graphs, and the filter.
   static constexpr int kDpGraphs = 8;
   GraphSegment g_dp[kDpGraphs], g_filter;
   uint64_t dp_kernels[kDpGraphs] = {};
-  int dp_next = 0;  // the entry that a ninth set replaces
+  int dp_next = 0;  // the entry that a ninth set takes over
   int64_t count = 0;
   int64_t in_count = 0;  // input pairs of the last run (the filter's scan covers them)
   bool valid = false;
@@ -222,6 +222,7 @@ struct crispy_ctx {
   void *h_hist = nullptr;  // pinned slot for small device read-backs
   bool timing = false;
   bool graphs = true;  // kernel chains through captured graphs (false: launched one by one)
+  uint64_t launches = 0, settled = 0;  // graph launches so far, and those known to have ended
   std::vector<PendingEvent> pending;
   std::vector<hipEvent_t> pool;
   std::map<std::string, KStat> stats;
@@ -242,6 +243,8 @@ void release(crispy_ctx *ctx, DevBuf &b);
 int ensure_host(crispy_ctx *ctx, size_t bytes);
 void timer_begin(crispy_ctx *ctx, const char *name, hipEvent_t *a, hipStream_t s = nullptr);
 void timer_end(crispy_ctx *ctx, const char *name, hipEvent_t a, double units, hipStream_t s = nullptr);
+// Waits for the main stream.
+int wait_main(crispy_ctx *ctx);
 int fork_workers(crispy_ctx *ctx);
 int join_workers(crispy_ctx *ctx);
 // NW timers: *units = the cells behind an NW DP timer name (summed on the

@@ -1,5 +1,4 @@
-// Captured launch sequences: a GraphSegment holds the instantiated graph of
-// one sequence and the arguments it was captured with.
+// Captured launch sequences.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -13,65 +12,84 @@ namespace crispy {
 
 inline void drop_segment(GraphSegment &g) {
   if (g.exec) (void)hipGraphExecDestroy(g.exec);
-  g.exec = nullptr;
-  g.key.clear();
+  g = GraphSegment();
 }
 
-// Runs enqueue(capturing) on the main stream through the segment's graph:
-// captured again when the key differs from the one it was captured with, and
-// then either applied to the instantiated graph in place (same launches, new
-// arguments: hipGraphExecUpdate) or instantiated anew.  A captured graph must
-// hold kernels and event dependencies only (memset nodes have given wrong
-// results on replays), which is checked.
+// The kernel functions of a captured graph's nodes, in node order (another
+// node's type in its place).  A graph must hold kernels and event dependencies
+// only: memset nodes, which have given wrong results on replays, are refused.
+inline int graph_kernels(crispy_ctx *ctx, hipGraph_t graph, const char *what, std::vector<const void *> *kernels) {
+  size_t nn = 0;
+  CRISPY_HIP(ctx, hipGraphGetNodes(graph, nullptr, &nn));
+  std::vector<hipGraphNode_t> nodes(nn);
+  if (nn) CRISPY_HIP(ctx, hipGraphGetNodes(graph, nodes.data(), &nn));
+  for (hipGraphNode_t node : nodes) {
+    hipGraphNodeType t;
+    CRISPY_HIP(ctx, hipGraphNodeGetType(node, &t));
+    if (t == hipGraphNodeTypeMemset)
+      return set_err(ctx, CRISPY_ERR_HIP, "capturing %s: the graph holds a memset node", what);
+    hipKernelNodeParams params = {};
+    if (t == hipGraphNodeTypeKernel) CRISPY_HIP(ctx, hipGraphKernelNodeGetParams(node, &params));
+    kernels->push_back(t == hipGraphNodeTypeKernel ? params.func : reinterpret_cast<const void *>((uintptr_t)t));
+  }
+  return CRISPY_OK;
+}
+
+// Runs enqueue(true) on the main stream, through the segment's graph where its
+// key comes a second time in a row: a program that repeats a run replays, one
+// whose runs all differ (a server's jobs) builds no graph at all.  A graph of
+// the same kernels takes over the instantiated one in place
+// (hipGraphExecUpdate with new arguments); one of other kernels replaces it.
+// Either way the last launch of the old one has ended first.  The key must
+// hold every argument of the launches, and which kernels they are must
+// determine their dependencies.
 template <class Enqueue>
 int run_segment(crispy_ctx *ctx, GraphSegment &g, std::vector<uintptr_t> key, const char *what,
                 Enqueue &&enqueue) {
   if (!ctx->graphs) return enqueue(false);
   if (!g.exec || key != g.key) {
+    if (key != g.seen) {
+      g.seen = std::move(key);
+      return enqueue(true);
+    }
     g.key.clear();
     CRISPY_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     const int rc = enqueue(true);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(ctx->stream, &graph);
-    if (rc != CRISPY_OK || e != hipSuccess) {
-      if (graph) (void)hipGraphDestroy(graph);
-      return rc != CRISPY_OK ? rc : set_err(ctx, CRISPY_ERR_HIP, "capturing %s: %s", what, hipGetErrorString(e));
-    }
-    size_t nn = 0;
-    hipError_t ge = hipGraphGetNodes(graph, nullptr, &nn);
-    std::vector<hipGraphNode_t> nodes(nn);
-    if (ge == hipSuccess && nn) ge = hipGraphGetNodes(graph, nodes.data(), &nn);
-    for (size_t k = 0; ge == hipSuccess && k < nn; ++k) {
-      hipGraphNodeType t;
-      ge = hipGraphNodeGetType(nodes[k], &t);
-      if (ge == hipSuccess && t == hipGraphNodeTypeMemset) {
-        (void)hipGraphDestroy(graph);
-        return set_err(ctx, CRISPY_ERR_HIP, "capturing %s: the graph holds a memset node", what);
+    struct Graph {
+      hipGraph_t g;
+      ~Graph() {
+        if (g) (void)hipGraphDestroy(g);
       }
-    }
-    if (ge != hipSuccess) {
-      (void)hipGraphDestroy(graph);
-      return set_err(ctx, CRISPY_ERR_HIP, "inspecting the %s graph: %s", what, hipGetErrorString(ge));
-    }
-    bool updated = false;
-    if (g.exec) {
+    } owner{graph};
+    if (rc != CRISPY_OK) return rc;
+    if (e != hipSuccess) return set_err(ctx, CRISPY_ERR_HIP, "capturing %s: %s", what, hipGetErrorString(e));
+    std::vector<const void *> kernels;
+    CRISPY_TRY(graph_kernels(ctx, graph, what, &kernels));
+    if (g.exec && g.launch > ctx->settled) CRISPY_TRY(wait_main(ctx));
+    if (g.exec && kernels == g.kernels) {
       hipGraphNode_t bad = nullptr;
       hipGraphExecUpdateResult ur = hipGraphExecUpdateError;
-      updated = hipGraphExecUpdate(g.exec, graph, &bad, &ur) == hipSuccess && ur == hipGraphExecUpdateSuccess;
-      if (!updated) {
+      if (hipGraphExecUpdate(g.exec, graph, &bad, &ur) != hipSuccess || ur != hipGraphExecUpdateSuccess) {
         (void)hipGetLastError();
         drop_segment(g);
       }
+    } else {
+      drop_segment(g);
     }
-    const hipError_t ie = updated ? hipSuccess : hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (ie != hipSuccess) {
-      g.exec = nullptr;
-      return set_err(ctx, CRISPY_ERR_HIP, "instantiating the %s graph: %s", what, hipGetErrorString(ie));
+    if (!g.exec) {
+      const hipError_t ie = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
+      if (ie != hipSuccess) {
+        g.exec = nullptr;
+        return set_err(ctx, CRISPY_ERR_HIP, "instantiating the %s graph: %s", what, hipGetErrorString(ie));
+      }
     }
+    g.kernels = std::move(kernels);
     g.key = std::move(key);
   }
   CRISPY_HIP(ctx, hipGraphLaunch(g.exec, ctx->stream));
+  g.launch = ++ctx->launches;
   return CRISPY_OK;
 }
 

@@ -1817,7 +1817,7 @@ static int run_counted(crispy_ctx *ctx, int64_t &cap, DevBuf &keys, DevBuf *dist
     CRISPY_TRY(launch());
     unsigned long long c = 0;
     CRISPY_HIP(ctx, hipMemcpyAsync(&c, km.counter.p, sizeof c, hipMemcpyDeviceToHost, ctx->stream));
-    CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    CRISPY_TRY(wait_main(ctx));
     *count = (int64_t)c;
     if (*count <= cap) return CRISPY_OK;
     if (attempt == 0) cap = *count + *count / 8 + 1024;  // rerun with room for every entry
@@ -1841,7 +1841,7 @@ static int run_segmented(crispy_ctx *ctx, int64_t *count, F &&launch) {
     CRISPY_TRY(ensure(ctx, km.cand, sizeof(uint64_t) * kCandSegs * km.cand_seg_cap));
     CRISPY_TRY(launch());
     CRISPY_HIP(ctx, hipMemcpyAsync(st, km.seg_stat.p, sizeof st, hipMemcpyDeviceToHost, ctx->stream));
-    CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    CRISPY_TRY(wait_main(ctx));
     *count = (int64_t)st[0];
     if ((int64_t)st[1] <= km.cand_seg_cap) return CRISPY_OK;
     if (attempt == 0) km.cand_seg_cap = (int64_t)st[1] + (int64_t)st[1] / 8 + 256;  // room for every segment
@@ -1950,7 +1950,7 @@ int crispy_kmer_autotune(crispy_ctx *ctx, int K, float threshold, int repeats, i
     km.hash_buckets = st.second;
     double fastest = 1e300;
     for (int r = 0; r <= repeats; ++r) {  // the first run warms up (profiles, graphs, buffers)
-      CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      CRISPY_TRY(wait_main(ctx));
       const auto t0 = std::chrono::steady_clock::now();
       const int rc = crispy_kmer_run(ctx, K, threshold, 0, -1, nullptr);
       if (rc != CRISPY_OK) {
@@ -1958,7 +1958,7 @@ int crispy_kmer_autotune(crispy_ctx *ctx, int K, float threshold, int repeats, i
         km.hash_buckets = before.second;
         return rc;
       }
-      CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      CRISPY_TRY(wait_main(ctx));
       const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
       if (r > 0) fastest = std::min(fastest, sec);
     }
@@ -2090,7 +2090,7 @@ static int kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
       CRISPY_TRY(refine_candidates(ctx, ncand, (double)pairs_in_range, threshold, K - 6));
       unsigned long long c = 0;
       CRISPY_HIP(ctx, hipMemcpyAsync(&c, km.cand_n.p, sizeof c, hipMemcpyDeviceToHost, ctx->stream));
-      CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      CRISPY_TRY(wait_main(ctx));
       nref = (int64_t)c;
     }
     // (i, j) order, so the lanes of a wave merge against the same few row lists
@@ -2170,7 +2170,7 @@ int crispy_kmer_fetch(crispy_ctx *ctx, int64_t first, int64_t count, int32_t *pa
   if (dists)
     CRISPY_HIP(ctx, hipMemcpyAsync(dists, km.dists_alt.as<float>() + first, sizeof(float) * count,
                                    hipMemcpyDeviceToHost, ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   return CRISPY_OK;
 }
 

@@ -523,10 +523,9 @@ static PkPlan pk_plan(int cus, int64_t np, int band, int maxlen, int kb_lo, int 
 
 // The DP phase's launches after the bucket sort: the plan, then every family
 // that the reads' kB range allows on its worker stream.  No host read-back and nothing sized by the histogram, so the
-// sequence can be captured into a graph.  Per-family timers only when not
-// capturing.
+// sequence can be captured into a graph.  Per-family timers only with graphs off.
 static int enqueue_dp(crispy_ctx *ctx, const NwFusedArgs &args, const unsigned (&grid)[kNumFamilies],
-                      const PkPlan &pk, bool capturing) {
+                      const PkPlan &pk, bool graphs) {
   NwState &nw = ctx->nw;
   nw_plan_kernel<<<1, 1024, 0, ctx->stream>>>(nw.hist.as<unsigned int>(), nw.cells.as<unsigned long long>(),
                                               pk.map, nw.plan.as<NwPlan>(),
@@ -538,13 +537,13 @@ static int enqueue_dp(crispy_ctx *ctx, const NwFusedArgs &args, const unsigned (
     hipStream_t s = ctx->workers[family_worker(f)];
     const char *name = f >= kFirstPkFamily ? "nw_band_pk" : f >= kNumRegFamilies ? "nw_band_sliced" : "nw_band_reg";
     hipEvent_t ev = nullptr;
-    if (!capturing) timer_begin(ctx, name, &ev, s);
+    if (!graphs) timer_begin(ctx, name, &ev, s);
     if (f >= kFirstPkFamily)
       kPkLaunch[f - kFirstPkFamily](s, grid[f], args, pk.args[f - kFirstPkFamily]);
     else
       kFamilyLaunch[f](s, grid[f], args);
     CRISPY_LAUNCHED(ctx);
-    if (!capturing) timer_end(ctx, name, ev, 0.0, s);
+    if (!graphs) timer_end(ctx, name, ev, 0.0, s);
   }
   return join_workers(ctx);
 }
@@ -660,21 +659,19 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   if (gi == NwState::kDpGraphs) {
     gi = nw.dp_next;
     nw.dp_next = (nw.dp_next + 1) % NwState::kDpGraphs;
-    CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));  // its last launch has ended
-    drop_segment(nw.g_dp[gi]);
   }
   nw.dp_kernels[gi] = kernels;
   hipEvent_t phase;
   timer_begin(ctx, "nw_dp_phase", &phase);
   CRISPY_TRY(run_segment(ctx, nw.g_dp[gi], std::move(key), "NW DP phase",
-                         [&](bool capturing) { return enqueue_dp(ctx, args, grid, pk, capturing); }));
+                         [&](bool graphs) { return enqueue_dp(ctx, args, grid, pk, graphs); }));
   // Pairs for the generic kernel: their count comes back from the plan, and it
   // runs after the families.
   if (maybe_generic) {
     uint2 *h_g = reinterpret_cast<uint2 *>(ctx->h_hist);
     CRISPY_HIP(ctx, hipMemcpyAsync(h_g, &plan->btab[kGenericBucket], sizeof(uint2), hipMemcpyDeviceToHost,
                                    ctx->stream));
-    CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    CRISPY_TRY(wait_main(ctx));
     nw.busy = false;  // the families are done
     const uint2 gb = *h_g;
     const int64_t ng = gb.y;
@@ -732,7 +729,7 @@ static int nw_filter(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, float thr
   timer_end(ctx, "nw_filter", ev, (double)np);
   unsigned int *h_c = reinterpret_cast<unsigned int *>(ctx->h_hist);
   CRISPY_HIP(ctx, hipMemcpyAsync(h_c, nw.nsel.p, sizeof *h_c, hipMemcpyDeviceToHost, ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   *count = *h_c;
   return CRISPY_OK;
 }
@@ -774,7 +771,7 @@ int nw_timer_units(crispy_ctx *ctx, const char *name, double *units) {
   unsigned long long *h = reinterpret_cast<unsigned long long *>(ctx->h_hist);
   CRISPY_HIP(ctx, hipMemcpyAsync(h, nw.stat.p, sizeof(unsigned long long) * (kNumFamilies + 1),
                                  hipMemcpyDeviceToHost, ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   for (int f = lo; f < hi; ++f) *units += (double)h[f];
   return CRISPY_OK;
 }
@@ -782,7 +779,7 @@ int nw_timer_units(crispy_ctx *ctx, const char *name, double *units) {
 int nw_timer_reset(crispy_ctx *ctx) {
   if (!ctx->nw.stat.p) return CRISPY_OK;
   CRISPY_HIP(ctx, hipMemsetAsync(ctx->nw.stat.p, 0, ctx->nw.stat.bytes, ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   return CRISPY_OK;
 }
 
@@ -950,7 +947,7 @@ int crispy_nw_fetch(crispy_ctx *ctx, int64_t first, int64_t count, int32_t *pair
   if (dists)
     CRISPY_HIP(ctx, hipMemcpyAsync(dists, nw.out_dists.as<float>() + first, sizeof(float) * count,
                                    hipMemcpyDeviceToHost, ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   return CRISPY_OK;
 }
 
@@ -969,7 +966,7 @@ int crispy_nw_file_split(crispy_ctx *ctx, int64_t chunk_pairs, int64_t flush_pai
     for (int64_t c = 0; c + 1 < chunks; ++c)
       CRISPY_HIP(ctx, hipMemcpyAsync(&ends[(size_t)c], nw.sel.as<uint32_t>() + (c + 1) * chunk_pairs,
                                      sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-    CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    CRISPY_TRY(wait_main(ctx));
     ends[(size_t)chunks - 1] = (uint32_t)nw.count;
   }
   int32_t f = 0;
@@ -1004,7 +1001,7 @@ int crispy_nw_fetch_sorted(crispy_ctx *ctx, int64_t first, int64_t count, int32_
   CRISPY_HIP(ctx, hipMemcpyAsync(pairs, nw.sort_pairs.p, sizeof(int2) * count, hipMemcpyDeviceToHost, ctx->stream));
   CRISPY_HIP(ctx, hipMemcpyAsync(dists, nw.sort_dists.p, sizeof(float) * count, hipMemcpyDeviceToHost,
                                  ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   return CRISPY_OK;
 }
 
@@ -1024,10 +1021,10 @@ int crispy_nw_autotune(crispy_ctx *ctx, int band, int repeats, int *chosen) {
     nw.slice_width = pol;
     double fastest = 1e300;
     for (int r = 0; r <= repeats; ++r) {  // the first run warms up
-      CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      CRISPY_TRY(wait_main(ctx));
       const auto t0 = std::chrono::steady_clock::now();
       CRISPY_TRY(nw_core(ctx, d, np, band));
-      CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      CRISPY_TRY(wait_main(ctx));
       const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
       if (r > 0) fastest = std::min(fastest, s);
     }
@@ -1076,7 +1073,7 @@ int crispy_nw_csr(crispy_ctx *ctx, int32_t n_rows, int64_t *row_ptr, int32_t *co
     CRISPY_HIP(ctx, hipMemcpyAsync(cols, nw.csr_cols.p, sizeof(int32_t) * c, hipMemcpyDeviceToHost, ctx->stream));
   if (c > 0 && vals)
     CRISPY_HIP(ctx, hipMemcpyAsync(vals, nw.out_dists.p, sizeof(float) * c, hipMemcpyDeviceToHost, ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   return CRISPY_OK;
 }
 
@@ -1123,7 +1120,7 @@ int crispy_nw_dists_noalloc(crispy_ctx *ctx, const int32_t *d_pairs, int64_t npa
   CRISPY_LAUNCHED(ctx);
   unsigned int *h_bad = reinterpret_cast<unsigned int *>(ctx->h_hist);
   CRISPY_HIP(ctx, hipMemcpyAsync(h_bad, bad, sizeof(unsigned int), hipMemcpyDeviceToHost, ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   if (*h_bad) return set_err(ctx, CRISPY_ERR_ARG, "a pair names a read outside [0, %d)", rs.n);
   nw_bucket_kernel<<<(int)std::min<int64_t>((npairs + 255) / 256, 1024), 256, 0, ctx->stream>>>(
       pairs, npairs, rs.len.as<int32_t>(), rs.clean.as<uint8_t>(), band, -1, bkey, keys, idx, hist, cells);
@@ -1143,7 +1140,7 @@ int crispy_nw_dists_noalloc(crispy_ctx *ctx, const int32_t *d_pairs, int64_t npa
     CRISPY_LAUNCHED(ctx);
   }
   CRISPY_TRY(join_workers(ctx));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   return CRISPY_OK;
 }
 
@@ -1156,7 +1153,7 @@ int crispy_nw_dists(crispy_ctx *ctx, const int32_t *pairs, int64_t npairs, int b
   if (npairs > 0)
     CRISPY_HIP(ctx, hipMemcpyAsync(dists, ctx->nw.dist.p, sizeof(float) * npairs, hipMemcpyDeviceToHost,
                                    ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   return CRISPY_OK;
 }
 
@@ -1179,7 +1176,7 @@ int crispy_sort_by_dist(crispy_ctx *ctx, int32_t *pairs, float *dists, int64_t n
                           nw.sort_pairs.as<int2>(), nw.sort_dists.as<float>()));
   CRISPY_HIP(ctx, hipMemcpyAsync(pairs, nw.sort_pairs.p, sizeof(int2) * n, hipMemcpyDeviceToHost, ctx->stream));
   CRISPY_HIP(ctx, hipMemcpyAsync(dists, nw.sort_dists.p, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
-  CRISPY_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  CRISPY_TRY(wait_main(ctx));
   return CRISPY_OK;
 }
 
