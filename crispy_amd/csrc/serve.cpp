@@ -60,7 +60,8 @@ struct Job {
   int K = 6, band = 10;
   float kthr = 0.f, nthr = 0.f;
   int64_t est = 0;
-  int64_t scratch = 0;  // charged beside `est`: the NW directions' allowance
+  int64_t want = 0;     // bytes the NW directions can use
+  int64_t scratch = 0;  // of them charged beside `est`
   int64_t held = 0;  // device bytes the slot's context held after the job
   // outgrew its charge while other jobs ran: queued again at the head,
   // charged the whole budget, so it runs alone
@@ -181,16 +182,23 @@ void worker_loop(crispy_server *srv, int slot) {
           // other slots hold
           const int64_t held = srv->charge[slot], sheld = crispy_ctx_scratch_bytes(ctx);
           const Job &head = *srv->queue.front();
-          // a job run again alone: one cap, the budget, over all its buffers
-          const int64_t scratch = head.solo ? 0 : std::max(sheld, head.scratch);
-          const int64_t need = head.solo ? std::max(held, head.est) : std::max(held - sheld, head.est) + scratch;
-          if (srv->reserved - held + need <= srv->budget) {
+          // A job is admitted by its estimate.  The directions take what that
+          // leaves of an even share of the rest of the budget over the slots
+          // without a job, so the next jobs still find theirs.  A job run again
+          // alone has one cap, the budget, over all its buffers.
+          const int64_t left = srv->budget - (srv->reserved - held);
+          const int64_t base = head.solo ? std::max(held, head.est) : std::max(held - sheld, head.est);
+          const int64_t share = left / ((int64_t)srv->ctxs.size() - srv->running);
+          const int64_t scratch = head.solo ? 0 : std::max({sheld, std::min(head.want, share - base), int64_t(0)});
+          const int64_t need = base + scratch;
+          if (need <= left) {
             job = srv->queue.front();
             srv->queue.pop_front();
             srv->reserved += need - held;
             srv->peak_reserved = std::max(srv->peak_reserved, srv->reserved);
             srv->charge[slot] = need;
             srv->running += 1;
+            job->scratch = scratch;
             if (!job->solo) job->t_start = Clock::now();
             // the job's buffers may not outgrow what it is charged
             crispy_ctx_set_mem_limit(ctx, need - scratch);
@@ -225,7 +233,6 @@ void worker_loop(crispy_server *srv, int slot) {
         // whole budget, before the jobs behind it
         job->solo = true;
         job->est = srv->budget;
-        job->scratch = 0;
         job->status = CRISPY_OK;
         job->error.clear();
         srv->put_block(std::move(job->res));
@@ -380,19 +387,15 @@ int64_t crispy_server_submit(crispy_server *srv, const char *kmer_bases, const i
   for (int32_t r = 0; r < n; ++r) lens.push_back(noff[r + 1] - noff[r]);
   std::lock_guard<std::mutex> lk(srv->mu);
   if (job->est > srv->budget) return CRISPY_ERR_NOMEM;  // would never be admitted
-  // What is left of an even share of the budget goes to what makes the job
-  // faster, so the slots still run side by side: a large K = 6 job's candidates,
-  // then the directions, 2 bits per band position and row.
-  {
-    if (K == 6 && (int64_t)n * (n - 1) / 2 >= kCandidatePairs &&
-        job->est + candidate_bytes(n) <= srv->budget / (int64_t)srv->ctxs.size())
-      job->est += candidate_bytes(n);
-    const int64_t len = n > 0 ? *std::max_element(lens.begin(), lens.end()) : 0;
-    const int64_t kb = band >= 2 ? len / band : len;
-    const double want = 1.5 * std::min<double>((double)n * (n - 1) / 2, 256.0 * n) * (len + 32) * (2 * kb + 32) / 4;
-    const int64_t share = srv->budget / (int64_t)srv->ctxs.size() - job->est;
-    job->scratch = std::max<int64_t>(0, std::min<int64_t>({share, int64_t(4) << 30, (int64_t)std::min(want, 1e12)}));
-  }
+  // a large K = 6 job takes candidates where an even share of the budget holds them
+  if (K == 6 && (int64_t)n * (n - 1) / 2 >= kCandidatePairs &&
+      job->est + candidate_bytes(n) <= srv->budget / (int64_t)srv->ctxs.size())
+    job->est += candidate_bytes(n);
+  // directions: 2 bits per band position and row
+  const int64_t len = n > 0 ? *std::max_element(lens.begin(), lens.end()) : 0;
+  const int64_t kb = band >= 2 ? len / band : len;
+  const double want = 1.5 * std::min<double>((double)n * (n - 1) / 2, 256.0 * n) * (len + 32) * (2 * kb + 32) / 4;
+  job->want = (int64_t)std::min(want, (double)(int64_t(4) << 30));
   job->id = srv->next_id++;
   job->t_submit = Clock::now();
   srv->jobs[job->id] = job;
