@@ -423,8 +423,8 @@ static int family_worker(int f) { return f % kNumWorkers; }
 // waves or `room` bytes hold, and its cost: the longer of one wave's task and
 // the chip's share of all tasks plus most of a last one, in instructions of
 // (rows + 2 lanes) steps of ~35 + 10.5 per cell, for kB evenly spread.
-static double pk_plan_cap(int cus, int64_t np, int band, int maxlen, int kb_lo, int kb_hi, int forced, int64_t room,
-                          int cap, PkPlan &p) {
+static double pk_plan_cap(int cus, int64_t np, int band, int maxlen, int kb_lo, int kb_hi, int forced, bool ext,
+                          int64_t room, int cap, PkPlan &p) {
   p = PkPlan();
   p.map = NwMap{forced, -1, cap};
   // a pair's rows: its shorter read, at most (L1 + L2) / 2 < band (kB + 1)
@@ -472,7 +472,7 @@ static double pk_plan_cap(int cus, int64_t np, int band, int maxlen, int kb_lo, 
       unsigned &b = p.slots[f];
       if (pass == 0)
         b = (unsigned)std::min((task_grid(np, per[f], buckets[f]) + kPkBlockWaves - 1) / kPkBlockWaves * kPkBlockWaves,
-                               (int64_t)4 * cus * kPkFamilies[f].waves);
+                               (int64_t)4 * cus * (ext ? kPkFamilies[f].ext_waves : kPkFamilies[f].waves));
       else
         b = (unsigned)(b * ((double)room / (double)full)) / kPkBlockWaves * kPkBlockWaves;
       if (!b) return 0;  // no room for a slot of every family
@@ -498,7 +498,8 @@ static double pk_plan_cap(int cus, int64_t np, int band, int maxlen, int kb_lo, 
 // 0.64 ms for 1.33.
 // Where the scratch is short of a wave per SIMD the unpacked kernels (~1.6x
 // the instructions, no scratch) are the faster ones.
-static PkPlan pk_plan(int cus, int64_t np, int band, int maxlen, int kb_lo, int kb_hi, int forced, int64_t room) {
+static PkPlan pk_plan(int cus, int64_t np, int band, int maxlen, int kb_lo, int kb_hi, int forced, bool ext,
+                      int64_t room) {
   PkPlan none, best;
   none.map = best.map = NwMap{forced, -1, kPkMaxCells};
   if (np == 0) return none;
@@ -507,12 +508,12 @@ static PkPlan pk_plan(int cus, int64_t np, int band, int maxlen, int kb_lo, int 
   int top = -1;
   for (int cap : {kPkMaxCells, 32, 24, 20, 16, 12, 8}) {
     PkPlan p;
-    const double unbounded = pk_plan_cap(cus, np, band, maxlen, kb_lo, kb_hi, forced, INT64_MAX, cap, p);
+    const double unbounded = pk_plan_cap(cus, np, band, maxlen, kb_lo, kb_hi, forced, ext, INT64_MAX, cap, p);
     if (!unbounded || p.map.pk_top < top) break;  // narrower slices reach fewer kB
     top = p.map.pk_top;
     if (!free_cost || unbounded < free_cost) free_cost = unbounded;
     const double cost = p.bytes() <= room ? unbounded
-                                          : pk_plan_cap(cus, np, band, maxlen, kb_lo, kb_hi, forced, room, cap, p);
+                                          : pk_plan_cap(cus, np, band, maxlen, kb_lo, kb_hi, forced, ext, room, cap, p);
     if (cost && (!best_cost || cost < best_cost)) {
       best_cost = cost;
       best = p;
@@ -594,7 +595,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   const int64_t room = ctx->scratch_limit >= 0 ? ctx->scratch_limit
                        : ctx->mem_limit > 0    ? ctx->mem_limit - ctx->dev_bytes + (int64_t)nw.dirs.bytes - later
                                                : kPkScratchBytes;
-  PkPlan pk = pk_plan(ctx->cus, np, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, room);
+  PkPlan pk = pk_plan(ctx->cus, np, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, rs.ext, room);
   struct Busy {
     NwState &nw;
     ~Busy() { nw.busy = false; }
@@ -603,7 +604,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
     const int rc = ensure(ctx, nw.dirs, (size_t)pk.bytes());
     if (rc == CRISPY_ERR_NOMEM) {  // a device that others fill: the unpacked kernels need no scratch
       ctx->err.clear();
-      pk = pk_plan(ctx->cus, 0, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, 0);
+      pk = pk_plan(ctx->cus, 0, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, rs.ext, 0);
     } else if (rc != CRISPY_OK) {
       return rc;
     }

@@ -1,5 +1,8 @@
-"""The packed NW kernels' scratch next to the generic kernel's, under a memory
-limit that holds the call without the former."""
+"""The packed NW kernels' direction scratch: next to the generic kernel's under a
+memory limit that holds the call without it, and no larger than the waves that
+the chip holds."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -41,3 +44,25 @@ def test_packed_and_generic_pairs_share_a_limit(slack):
             print("slack", slack, flush=True)
             assert np.array_equal(c.nw_dists(pairs, 1), want)
             assert c.device_bytes() <= need + slack
+
+
+def test_reads_with_other_bytes_take_slots_for_their_waves():
+    """Their kernels run fewer waves per SIMD (4 for 5 at these widths), so a
+    call that fills the chip needs as many fewer direction slots."""
+    rng = np.random.default_rng(5)
+    plain = _reads(rng.integers(60, 101, 400), 6)
+    bases = bytearray(plain.bases)
+    bases[int(plain.offsets[200]) + 7] = ord("N")
+    ambiguous = ca.Reads(bytes(bases), plain.offsets)
+    pairs = rng.integers(0, plain.n, (800000, 2)).astype(np.int32)
+    held, got = [], []
+    for reads in (plain, ambiguous):
+        with ca.Context(0) as c:
+            c._L.crispy_ctx_scratch_bytes.restype = ctypes.c_int64
+            c.upload_reads(ca.NW, reads)
+            got.append(c.nw_dists(pairs, 10))
+            held.append(c._L.crispy_ctx_scratch_bytes(c._h))
+    print(held, flush=True)
+    assert 0 < held[1] <= 0.8 * held[0] + 1
+    clean = (pairs != 200).all(1)
+    assert np.array_equal(got[0][clean], got[1][clean])
