@@ -1,6 +1,6 @@
 """The packed NW kernels' direction scratch: next to the generic kernel's under a
-memory limit that holds the call without it, and no larger than the waves that
-the chip holds."""
+memory limit that holds the call without it, no larger than the waves that the
+chip holds, and smaller than a call wants; and next to forced slice widths."""
 import ctypes
 
 import numpy as np
@@ -66,3 +66,61 @@ def test_reads_with_other_bytes_take_slots_for_their_waves():
     assert 0 < held[1] <= 0.8 * held[0] + 1
     clean = (pairs != 200).all(1)
     assert np.array_equal(got[0][clean], got[1][clean])
+
+
+# lengths, pairs, band, other bytes: one family to each worker, two to each,
+# several lanes per pair, the kernels for other bytes
+SHORT = {
+    "two families": (100, 230, 300000, 10, False),
+    "four families": (150, 550, 150000, 10, False),
+    "several lanes": (100, 320, 30000, 2, False),
+    "other bytes": (100, 230, 300000, 10, True),
+}
+
+
+@pytest.mark.parametrize("name", list(SHORT))
+def test_fewer_slots_than_wanted(name):
+    """A scratch of a part of what the call takes without a limit: fewer
+    direction slots, each for several tasks; and one too small for any."""
+    lo, hi, npairs, band, other = SHORT[name]
+    rng = np.random.default_rng(7)
+    reads = _reads(rng.integers(lo, hi + 1, 500), 8)
+    if other:
+        bases = bytearray(reads.bases)
+        for r in range(0, reads.n, 3):
+            bases[int(reads.offsets[r]) + 9] = ord("N")
+        reads = ca.Reads(bytes(bases), reads.offsets)
+    pairs = rng.integers(0, reads.n, (npairs, 2)).astype(np.int32)
+    with ca.Context(0) as c:
+        c._L.crispy_ctx_scratch_bytes.restype = ctypes.c_int64
+        c._L.crispy_ctx_set_scratch_limit.argtypes = [ctypes.c_void_p, ctypes.c_int64]
+        c.upload_reads(ca.NW, reads)
+        want = c.nw_dists(pairs, band)
+        full = c._L.crispy_ctx_scratch_bytes(c._h)
+    assert full > 0
+    for part in (0.9, 0.6, 0.4, 0.0005):
+        with ca.Context(0) as c:
+            limit = int(part * full)
+            c._check(c._L.crispy_ctx_set_scratch_limit(c._h, limit))
+            c.upload_reads(ca.NW, reads)
+            print(name, part, limit, flush=True)
+            for _ in range(3):
+                assert np.array_equal(c.nw_dists(pairs, band), want)
+            held = c._L.crispy_ctx_scratch_bytes(c._h)
+            assert 0.9 * limit <= held <= limit if part > 0.1 else held == 0
+
+
+@pytest.mark.parametrize("band", [2, 5])
+def test_forced_slice_widths(band):
+    """Half bands up to 32 run packed, wider ones in the forced sliced kernel."""
+    rng = np.random.default_rng(9)
+    reads = _reads(rng.integers(40, 321, 200), 10)
+    pairs = rng.integers(0, reads.n, (20000, 2)).astype(np.int32)
+    with ca.Context(0) as c:
+        c.upload_reads(ca.NW, reads)
+        want = c.nw_dists(pairs, band)
+        for width in (24, 32, 0):
+            c.nw_slice_width(width)
+            for _ in range(3):
+                print("band", band, "width", width, flush=True)
+                assert np.array_equal(c.nw_dists(pairs, band), want)
