@@ -19,28 +19,20 @@ int set_err(crispy_ctx *ctx, int code, const char *fmt, ...) {
 }
 
 // Frees what the context can do without, so that it never keeps buffer b from
-// growing: the NW directions' scratch (if `dirs`), the upper code bits of
-// reads with other bytes, whose pairs then take the slower kernels, and the
-// candidate buffers of the last k-mer run.  Not what a run in preparation
-// uses.  True if something was freed.
+// growing: the NW directions' scratch (if `dirs`) and the upper code bits of
+// reads with other bytes, whose pairs then take the slower kernels.  Not while
+// an NW phase in preparation uses them.  True if something was freed.
 static bool make_room(crispy_ctx *ctx, const DevBuf &b, bool dirs) {
-  KmerState &km = ctx->km;
-  NwState &nw = ctx->nw;
   ReadStore &rs = ctx->reads[CRISPY_READS_NW];
-  if (&b == &nw.dirs) return false;
-  std::vector<DevBuf *> spare;
-  if (!nw.busy) {
-    if (dirs) spare.push_back(&nw.dirs);
-    spare.push_back(&rs.pack_hi);
+  dirs = dirs && ctx->nw.dirs.p;
+  const bool hi = &b != &rs.pack_hi && rs.pack_hi.p;
+  if (&b == &ctx->nw.dirs || ctx->nw.busy || !(dirs || hi)) return false;
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+  if (dirs) release(ctx, ctx->nw.dirs);
+  if (hi) {
+    release(ctx, rs.pack_hi);
+    rs.ext = false;
   }
-  if (!km.busy)
-    spare.insert(spare.end(), {&km.cand, &km.cand_alt, &km.cand_n, &km.seg, &km.seg_stat, &km.hbitmap, &km.hexcess,
-                               &km.hbound});
-  spare.erase(std::remove_if(spare.begin(), spare.end(), [&](const DevBuf *d) { return !d->p || d == &b; }),
-              spare.end());
-  if (spare.empty() || hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
-  for (DevBuf *d : spare) release(ctx, *d);
-  rs.ext = rs.ext && rs.pack_hi.p;
   return true;
 }
 

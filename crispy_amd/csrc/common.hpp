@@ -150,7 +150,6 @@ struct KmerState {
   int64_t cap = 0;
   int64_t count = 0;
   int32_t reads = 0;  // the read count that the result's pairs lie in
-  bool busy = false;  // a run uses its candidate buffers (hashed bitmaps, segments): not freed to make room
   bool valid = false;
   GraphSegment g_profile, g_tile;  // captured profile pass and tile pass
 };

@@ -287,9 +287,7 @@ constexpr int kCandPopShift = 44;
 constexpr int kCandWin = 32;
 constexpr int kListSlack = 32;
 static_assert(kCandWin % 4 == 0 && kCandWin <= kListSlack, "a window starts on a word at or before the list's last code");
-// Pairs from which the K <= 6 exact counts run as a pass of their own (auto
-// mode): k = 6 (hashed sweep), and K < 6 (tiles on the exact bitmaps).
-constexpr int64_t kExactPassPairs6 = 400000000;
+// Pairs from which the K <= 6 exact counts run as a pass of their own (auto mode).
 constexpr int64_t kExactPassPairs = 1000000000;
 constexpr uint64_t kCandKeyMask = (1ull << 40) - 1;
 
@@ -1975,9 +1973,9 @@ int crispy_kmer_autotune(crispy_ctx *ctx, int K, float threshold, int repeats, i
   return CRISPY_OK;
 }
 
-// crispy_kmer_run; `in_tile`: K <= 6 counts in the tile whatever the pair count.
-static int kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin, int64_t tile_end, int64_t *count,
-                    bool in_tile) {
+int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin, int64_t tile_end,
+                    int64_t *count) {
+  if (!ctx) return CRISPY_ERR_ARG;
   if (K < 1 || K > 8) return set_err(ctx, CRISPY_ERR_ARG, "unsupported K=%d (1..8)", K);
   CRISPY_HIP(ctx, hipSetDevice(ctx->device));
   ReadStore &rs = ctx->reads[CRISPY_READS_KMER];
@@ -2007,20 +2005,13 @@ static int kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
   while ((1 << km.kshift) < n) ++km.kshift;
   const int KP = K <= 6 ? K : 6;
   // K <= 6: exact counts in the tile, or in a pass of their own over the
-  // tile's candidates.  Measured per k-mer run at k = 6, 150-550 bp, counts in
-  // the tile against the hashed sweep and the pass: 12,000 reads 0.48 and
-  // 0.66 ms, 20,000 0.78 and 0.87, 30,000 1.28 and 1.19, 45,000 2.34 and
-  // 1.71, 60,000 3.87 and 2.31; below, the extra passes' launches and
-  // latency-bound merges cost more than the sweep saves.  K < 6 runs its
-  // candidate tiles on the exact bitmaps, which win from ~10^9 pairs up.
+  // tile's candidates (k = 6: the hashed sweep's).  Which is faster depends on
+  // how many pairs pass, which is not known before.  Counts in the tile against
+  // the passes, k = 6, reads of 200-300 bp: 30,000 reads, 0.01 % pass 1.03 and
+  // 0.57 ms, 1.5 % 1.65 and 2.04, 15 % 5.1 and 12.8; 100,000 reads, 0.01 % 8.4 and
+  // 2.7, 0.75 % 12.1 and 11.9.  So the passes start at 10^9 pairs.
   // exact_pass 2: the candidate form on the exact bitmaps (no hashing).
-  const bool separate = km.exact_pass >= 1 || (km.exact_pass == -1 && !in_tile &&
-                         (int64_t)n * (n - 1) / 2 >= (K == 6 ? kExactPassPairs6 : kExactPassPairs));
-  struct Busy {
-    KmerState &km;
-    ~Busy() { km.busy = false; }
-  } busy{km};
-  km.busy = K > 6 || separate;
+  const bool separate = km.exact_pass >= 1 || (km.exact_pass == -1 && (int64_t)n * (n - 1) / 2 >= kExactPassPairs);
   CRISPY_TRY(build_profiles(ctx, KP, K, (K > 6 || separate) && km.exact_pass != 2));
   // the k = 6 candidate tiles: on the hashed bitmaps, or on the exact ones
   const TileFn tiles6 = !km.hashed                          ? launch_tiles<6, true>
@@ -2125,7 +2116,6 @@ static int kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
       return CRISPY_OK;
     }));
   }
-  km.busy = false;
   CRISPY_TRY(ensure(ctx, km.keys_alt, sizeof(uint64_t) * (km.count + 1)));
   CRISPY_TRY(ensure(ctx, km.dists_alt, sizeof(float) * (km.count + 1)));
   CRISPY_TRY(ensure(ctx, km.pairs, sizeof(int2) * (km.count + 1)));
@@ -2140,20 +2130,6 @@ static int kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin,
   km.valid = true;
   if (count) *count = km.count;
   return CRISPY_OK;
-}
-
-int crispy_kmer_run(crispy_ctx *ctx, int K, float threshold, int64_t tile_begin, int64_t tile_end,
-                    int64_t *count) {
-  if (!ctx) return CRISPY_ERR_ARG;
-  const int rc = kmer_run(ctx, K, threshold, tile_begin, tile_end, count, false);
-  const int64_t n = ctx->reads[CRISPY_READS_KMER].n, pairs = n * (n - 1) / 2;
-  // No room for the candidates: counts in the tile need none (from
-  // kExactPassPairs up they would take several times as long).
-  if (rc != CRISPY_ERR_NOMEM || K != 6 || ctx->km.exact_pass != -1 || pairs < kExactPassPairs6 ||
-      pairs >= kExactPassPairs)
-    return rc;
-  ctx->err.clear();
-  return kmer_run(ctx, K, threshold, tile_begin, tile_end, count, true);
 }
 
 int crispy_kmer_fetch(crispy_ctx *ctx, int64_t first, int64_t count, int32_t *pairs, float *dists) {

@@ -257,9 +257,8 @@ void worker_loop(crispy_server *srv, int slot) {
 // Widest half band kB = (L1 + L2) / (2 band) the register and sliced NW
 // kernels take (64 lanes x 24 cells per pair); wider pairs use the generic one.
 constexpr int64_t kSlicedMaxHalfBand = (64 * 24 - 1) / 2;
-// K = 6 jobs of this many pairs take hashed candidates if there is room
-// (kExactPassPairs6 in kmer.hip).
-constexpr int64_t kCandidatePairs = 400000000;
+// K <= 6 jobs of this many pairs take candidates (kExactPassPairs in kmer.hip).
+constexpr int64_t kCandidatePairs = 1000000000;
 
 // First size of the k-mer result: the pairs in the tiles, at most 4 Mi.
 int64_t result_guess(int32_t n) {
@@ -387,7 +386,7 @@ int64_t crispy_server_submit(crispy_server *srv, const char *kmer_bases, const i
   for (int32_t r = 0; r < n; ++r) lens.push_back(noff[r + 1] - noff[r]);
   std::lock_guard<std::mutex> lk(srv->mu);
   if (job->est > srv->budget) return CRISPY_ERR_NOMEM;  // would never be admitted
-  // a large K = 6 job takes candidates where an even share of the budget holds them
+  // a large K = 6 job is charged its candidates where an even share of the budget holds them
   if (K == 6 && (int64_t)n * (n - 1) / 2 >= kCandidatePairs &&
       job->est + candidate_bytes(n) <= srv->budget / (int64_t)srv->ctxs.size())
     job->est += candidate_bytes(n);

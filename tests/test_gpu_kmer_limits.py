@@ -1,6 +1,8 @@
-"""Large k = 6 runs (from 4 x 10^8 pairs up, which take candidates) where
-memory holds the counts in the tile only: the same pairs and distances, in a
-context with a limit and in a server with a budget."""
+"""A k = 6 run of 4 x 10^8 pairs where memory holds counts in the tile only, in a
+context with a limit and in a server with a budget; and the time of a run most
+of whose pairs pass."""
+import time
+
 import numpy as np
 import pytest
 
@@ -54,24 +56,6 @@ def test_limit_that_holds_the_counts_in_the_tile(reads, in_tile):
             print("limit", need, flush=True)
             assert _same(_job(c, reads), want)
             assert c.device_bytes() <= need
-        c.mem_limit(0)  # candidates again
-        assert _same(_job(c, reads), want)
-        assert c.kmer_tile_bits() == 1280
-
-
-def test_candidates_make_room_for_the_pairs(reads, in_tile):
-    """A limit that holds the k-mer run's candidates, then not the NW stage's
-    buffers beside them."""
-    want, need = in_tile
-    with ca.Context(0) as c:
-        c.upload_reads(ca.KMER, reads)
-        c.kmer_run(6, THR)
-        assert c.kmer_tile_bits() == 1280
-    with ca.Context(0) as c:
-        c.mem_limit(need + (24 << 20))
-        for _ in range(2):
-            print("limit", need + (24 << 20), flush=True)
-            assert _same(_job(c, reads), want)
 
 
 def test_budget_that_holds_the_counts_in_the_tile(reads, in_tile):
@@ -84,3 +68,26 @@ def test_budget_that_holds_the_counts_in_the_tile(reads, in_tile):
             jid = srv.submit(reads, 6, THR, BAND, THR)
             assert _same(srv.fetch(jid), want[2:])
         assert srv.status()["peak_reserved_bytes"] <= budget
+
+
+def test_dense_run_takes_no_longer_than_counts_in_the_tile(reads):
+    """A fifth of all pairs pass: with candidates the run took 2.5 times as long."""
+    rng = np.random.default_rng(2)
+    codes = rng.integers(0, 4, (5, 250))[rng.integers(0, 5, N)]
+    hit = rng.random(codes.shape) < 0.02
+    codes[hit] = rng.integers(0, 4, int(hit.sum()))
+    dense = ca.Reads(np.frombuffer(b"ACGT", np.uint8)[codes].tobytes(), np.arange(N + 1, dtype=np.int64) * 250)
+    times = {}
+    for mode in (0, -1):
+        with ca.Context(0) as c:
+            c.upload_reads(ca.KMER, dense)
+            c.kmer_exact_pass(mode)
+            best = 1e9
+            for _ in range(6):
+                t0 = time.perf_counter()
+                assert c.kmer_run(6, 0.2) > 0.15 * N * (N - 1) / 2
+                c.sync()
+                best = min(best, time.perf_counter() - t0)
+        times[mode] = best
+    print(times, flush=True)
+    assert times[-1] < 1.5 * times[0]
