@@ -399,13 +399,22 @@ static int64_t family_grid(int f, int64_t np, int kb_lo, int kb_hi, const NwMap 
   return buckets ? task_grid(np, per, buckets) : 0;
 }
 
+// Stream of family f: the worker streams, and the main one (kMainStream) between
+// their fork and join.  Neighbouring families, which common length spreads put
+// to work together, run side by side, and the packed families beside the sliced
+// ones that take a call's wider bands.
+constexpr int kMainStream = kNumWorkers, kNumStreams = kNumWorkers + 1;
+static int family_stream(int f) { return f >= kFirstPkFamily && f % 2 == 0 ? kMainStream : f % kNumWorkers; }
+static_assert(kNumWorkers == 2 && kFirstPkFamily % 2 == 0, "packed families alternate: main stream, second worker");
+
 // The packed families' part of one DP phase: which kB they take, and per
 // family the waves (= direction slots) and their scratch.
 struct PkPlan {
   NwMap map;
   unsigned slots[kNumPkFamilies] = {};
   PkLaunchArgs args[kNumPkFamilies] = {};
-  int64_t region[kNumWorkers] = {};  // scratch bytes of each worker stream: its families run one after the other
+  int64_t region[kNumStreams] = {};  // scratch bytes of each stream: its families run one after the other
+  bool beside = false;               // a small part of the call, done well before the sliced kernels' (pk_plan)
   int64_t bytes() const {
     int64_t b = 0;
     for (int64_t r : region) b += r;
@@ -415,44 +424,108 @@ struct PkPlan {
 // Direction scratch of one context, at most.
 constexpr int64_t kPkScratchBytes = int64_t(4) << 30;
 
-// Worker stream of family f (neighbouring families, which common length
-// spreads put to work together, run side by side).
-static int family_worker(int f) { return f % kNumWorkers; }
+// What a DP phase takes, in us: its latency (the families of a worker stream run
+// one after the other, each at least as long as its longest wave task) against
+// the chip's time for all tasks and most of a last one.  The constants are
+// fitted to the phase's time over 776 calls: 11 ranges of lengths from 20-40 to
+// 1,500-2,048 bp, 9 bands, 1 to 1.5 M pairs, each in the unpacked kernels and in
+// packed slices of 40 to 8 cells (see pk_plan for how well they choose).
+struct DpCost {
+  double longest[kNumFamilies] = {};
+  double issue = 0;  // of all tasks on one SIMD
 
-// A plan with slices of at most `cap` cells, as many slots as the chip holds
-// waves or `room` bytes hold, and its cost: the longer of one wave's task and
-// the chip's share of all tasks plus most of a last one, in instructions of
-// (rows + 2 lanes) steps of ~35 + 10.5 per cell, for kB evenly spread.
-static double pk_plan_cap(int cus, int64_t np, int band, int maxlen, int kb_lo, int kb_hi, int forced, bool ext,
-                          int64_t room, int cap, PkPlan &p) {
-  p = PkPlan();
-  p.map = NwMap{forced, -1, cap};
+  // `pairs` pairs of bucket kb with up to `rows` rows
+  void add(int kb, int rows, double pairs, const NwMap &map) {
+    const int f = nw_family_of(kb, map), W = 2 * kb + 1;
+    // steps in the boundary's and in the last column's form, as parts of all
+    auto edge = [&](int lag) {
+      return std::min(1.0, (double)std::max(kb, lag) / rows) + std::min(1.0, (double)kb / rows);
+    };
+    double task, work;
+    int per_wave = 64;
+    if (f >= kFirstPkFamily) {
+      const int lanes = pk_lanes(kb, map.pk_cap), cells = pk_cells(kb, map.pk_cap), steps = rows + 2 * lanes;
+      per_wave = 64 / lanes;
+      const double e = edge(2 * lanes);
+      // the trace takes longer the more pairs a wave walks at once
+      task = steps * (0.313 + 0.06 * std::log2(1.0 + per_wave) + cells * (0.0245 + 0.0115 * e));
+      work = steps * (0.166 + cells * (0.0158 + 0.00468 * e));
+    } else if (f < kNumRegFamilies) {
+      const double e = edge(1);
+      task = rows * (0.109 + W * (0.02 + 0.00994 * e));
+      work = rows * W * (0.0164 + 0.00073 * e);
+    } else {
+      const int cells = kSliceWidths[f - kNumRegFamilies], lanes = slice_lanes(kb, cells), steps = rows + lanes;
+      per_wave = 64 / lanes;
+      const double e = edge(lanes);
+      task = steps * (0.228 + cells * (0.0214 + 0.00905 * e));
+      work = steps * cells * (0.0187 + 0.00721 * e);
+    }
+    longest[f] = std::max(longest[f], task);
+    issue += pairs / per_wave * work;
+  }
+
+  // `beside`: the streams with packed families end well before the others
+  double us(double simds, bool *beside) const {
+    double stream[kNumStreams] = {}, last = 0;
+    bool packed[kNumStreams] = {};
+    for (int f = 0; f < kNumFamilies; ++f) {
+      if (longest[f] == 0) continue;
+      stream[family_stream(f)] += longest[f] + 2.67;
+      packed[family_stream(f)] |= f >= kFirstPkFamily;
+      last = std::max(last, longest[f] * (f >= kFirstPkFamily ? 0.971 : f < kNumRegFamilies ? 0.849 : 0.52));
+    }
+    double most[2] = {};
+    for (int w = 0; w < kNumStreams; ++w) most[packed[w]] = std::max(most[packed[w]], stream[w]);
+    *beside = most[1] <= 0.8 * most[0];
+    const double latency = std::max(most[0], most[1]), busy = issue / simds + last;
+    const double l2 = latency * latency, b2 = busy * busy;
+    return std::sqrt(std::sqrt(l2 * l2 + b2 * b2));
+  }
+};
+
+// The reads and pairs of a call, as far as plans depend on them.
+struct DpShape {
+  int64_t np;
+  int band, maxlen, kb_lo, kb_hi, forced;
+  bool ext;
   // a pair's rows: its shorter read, at most (L1 + L2) / 2 < band (kB + 1)
-  auto rows = [&](int kb) { return (int)std::min<int64_t>(maxlen, band >= 2 ? (int64_t)band * (kb + 1) : kb); };
-  kb_lo = std::max(kb_lo, 0);
-  const int kb_end = std::min(kb_hi, forced ? kKbRegMax : kPkMaxKb);
-  for (int kb = kb_lo; kb <= kb_end && pk_keys_fit(kb, rows(kb), cap); ++kb) p.map.pk_top = kb;
+  int rows(int kb) const { return (int)std::min<int64_t>(maxlen, band >= 2 ? (int64_t)band * (kb + 1) : kb); }
+  // the cost of `map` on `simds` SIMDs, for kB evenly spread, of up to about 32
+  // of them (a host microsecond counts in the smallest calls)
+  double us(const NwMap &map, double simds, bool *beside) const {
+    DpCost c;
+    const int lo = std::max(kb_lo, 0), hi = std::min(kb_hi, kKbSliceMax), stride = std::max(1, (hi - lo + 1) / 32);
+    const double pairs = (double)np / (kb_hi - kb_lo + 1);
+    for (int kb = hi; kb >= lo; kb -= stride)
+      c.add(kb, std::max(rows(kb), 1), pairs * std::min(stride, kb - lo + 1), map);
+    return c.us(simds, beside);
+  }
+};
+
+// A plan with slices of at most `cap` cells, and as many slots as the chip
+// holds waves or `room` bytes hold; its cost, 0 if there is none.
+static double pk_plan_cap(int cus, const DpShape &q, int64_t room, int cap, PkPlan &p) {
+  p = PkPlan();
+  p.map = NwMap{q.forced, -1, cap};
+  const int kb_lo = std::max(q.kb_lo, 0), kb_end = std::min(q.kb_hi, q.forced ? kKbRegMax : kPkMaxKb);
+  for (int kb = kb_lo; kb <= kb_end && pk_keys_fit(kb, q.rows(kb), cap); ++kb) p.map.pk_top = kb;
   if (p.map.pk_top < 0) return 0;
-  double total = 0, longest = 0;
   int64_t per[kNumPkFamilies] = {}, buckets[kNumPkFamilies] = {};
-  const double pairs = (double)np / (p.map.pk_top - kb_lo + 1);
   for (int f = 0; f < kNumPkFamilies; ++f) {
     p.args[f].cap = cap;
     p.args[f].f16 = true;
   }
   for (int kb = kb_lo; kb <= p.map.pk_top; ++kb) {
-    const int lanes = pk_lanes(kb, cap), cells = pk_cells(kb, cap), steps = rows(kb) + 2 * lanes;
+    const int lanes = pk_lanes(kb, cap), cells = pk_cells(kb, cap), steps = q.rows(kb) + 2 * lanes;
     int f = 0;
     while (cells > kPkFamilies[f].hi) ++f;
     PkLaunchArgs &x = p.args[f];
     per[f] = per[f] ? std::min<int64_t>(per[f], 64 / lanes) : 64 / lanes;
     ++buckets[f];
-    x.f16 = x.f16 && pk_keys_fit(kb, rows(kb), cap, kPkF16Top);
+    x.f16 = x.f16 && pk_keys_fit(kb, q.rows(kb), cap, kPkF16Top);
     x.words = std::max<int64_t>(x.words, (int64_t)(steps + kPkTraceSteps - 1) / kPkTraceSteps * kPkTraceSteps *
                                              pk_dir_words(cells) * 64);
-    const double task = steps * (35 + 10.5 * cells);
-    total += pairs / (64 / lanes) * task;
-    longest = std::max(longest, task);
   }
   // Blocks of four waves, one per SIMD, where up to two families run: one-wave
   // blocks land unevenly (2,747 tasks put 2 to 4 on a SIMD, and the call ended
@@ -471,59 +544,74 @@ static double pk_plan_cap(int cus, int64_t np, int band, int maxlen, int kb_lo, 
       if (!p.args[f].words) continue;
       unsigned &b = p.slots[f];
       if (pass == 0)
-        b = (unsigned)std::min((task_grid(np, per[f], buckets[f]) + kPkBlockWaves - 1) / kPkBlockWaves * kPkBlockWaves,
-                               (int64_t)4 * cus * (ext ? kPkFamilies[f].ext_waves : kPkFamilies[f].waves));
+        b = (unsigned)std::min((task_grid(q.np, per[f], buckets[f]) + kPkBlockWaves - 1) / kPkBlockWaves * kPkBlockWaves,
+                               (int64_t)4 * cus * (q.ext ? kPkFamilies[f].ext_waves : kPkFamilies[f].waves));
       else
         b = (unsigned)(b * ((double)room / (double)full)) / kPkBlockWaves * kPkBlockWaves;
       if (!b) return 0;  // no room for a slot of every family
-      int64_t &r = p.region[family_worker(kFirstPkFamily + f)];
+      int64_t &r = p.region[family_stream(kFirstPkFamily + f)];
       r = std::max(r, 4 * (int64_t)b * p.args[f].words);
       slots += b;
     }
     full = p.bytes();
-    const double simds = (double)std::min<int64_t>(slots, 4 * cus);
-    const double cost = std::max(longest, total / simds + 0.9 * longest);
-    if (full <= room) return cost;
+    if (full <= room) {
+      const double us = q.us(p.map, pass == 0 ? 4 * cus : (double)std::min<int64_t>(slots, 4 * cus), &p.beside);
+      p.beside = p.beside && 9 * (p.map.pk_top - kb_lo + 1) < 4 * (q.kb_hi - kb_lo + 1);
+      return us;
+    }
     if (room <= 0) return 0;
   }
   return 0;
 }
 
-// Slice width: a wider slice has less of the instructions that each step
-// spends beside its cells, a narrower one splits few pairs over more waves and
-// needs less scratch; the cost above picks it.  Over 18 inputs from 123 to 3.3 M
-// pairs the pick was the fastest of the seven widths or within 3 % of it, twice
-// within 15 %; against 16 cells everywhere a step with 3.3 M pairs of 150-550 bp
-// takes 17.3 ms for 19.6, against 40 everywhere 200 pairs of 1 kbp take
-// 0.64 ms for 1.33.
-// Where the scratch is short of a wave per SIMD the unpacked kernels (~1.6x
-// the instructions, no scratch) are the faster ones.
-static PkPlan pk_plan(int cus, int64_t np, int band, int maxlen, int kb_lo, int kb_hi, int forced, bool ext,
-                      int64_t room) {
+// Slice width, and whether the call runs packed at all.  A wider slice has less
+// of the instructions that each step spends beside its cells, a narrower one
+// splits few pairs over more waves and needs less scratch.  The unpacked kernels
+// issue more, but have no directions to wait for and to trace: they are the
+// faster ones for few pairs of narrow bands, for reads whose keys fit 16 bits
+// only in part, and where the scratch is short.  The cost above decides.
+// Where the packed kernels take less than 4/9 of the kB range and end well
+// before the sliced ones beside them, the call is as long with them as without
+// (1.3-1.9 kbp at band 10, 500 and 2,000 pairs: 2.21 and 2.45 ms against 2.24 and
+// 2.40) and the cost, which counts their work too, a tenth too high.
+// Over 1,246 calls of band 2 and more (those that the cost was fitted to and nine
+// other ranges of lengths) the pick is within 3 % of the fastest of all on
+// average, and slower than the unpacked kernels by more than 5 % in 24, by 29 %
+// at most; with the packed kernels wherever the keys fit more than 400 were,
+// up to 3.4 times as long.  Whole calls so and now: 1,000 pairs of 30-60 bp at band
+// 20 118 -> 90 us, 30 pairs of 1.5-2 kbp at band 10 5.2 -> 2.1 ms, 1,000 of
+// 200-300 bp at band 5 0.39 -> 0.32 ms, 30 of 400-900 bp at band 2 1.54 -> 1.13 ms.
+// Pairs with other bytes, and full alignments, had the generic kernel, which
+// takes many times as long: they run packed as far as the widest slices reach,
+// unless the scratch is short of a wave per SIMD.
+static PkPlan pk_plan(int cus, const DpShape &q, int64_t room) {
   PkPlan none, best;
-  none.map = best.map = NwMap{forced, -1, kPkMaxCells};
-  if (np == 0) return none;
+  none.map = best.map = NwMap{q.forced, -1, kPkMaxCells};
+  if (q.np == 0) return none;
   room = std::min(room, kPkScratchBytes);
+  const bool all_packed = q.ext || q.band < 2;
   double best_cost = 0, free_cost = 0;
   int top = -1;
   for (int cap : {kPkMaxCells, 32, 24, 20, 16, 12, 8}) {
     PkPlan p;
-    const double unbounded = pk_plan_cap(cus, np, band, maxlen, kb_lo, kb_hi, forced, ext, INT64_MAX, cap, p);
-    if (!unbounded || p.map.pk_top < top) break;  // narrower slices reach fewer kB
+    const double unbounded = pk_plan_cap(cus, q, INT64_MAX, cap, p);
+    // narrower slices reach fewer kB
+    if (!unbounded || (all_packed && p.map.pk_top < top)) break;
     top = p.map.pk_top;
     if (!free_cost || unbounded < free_cost) free_cost = unbounded;
-    const double cost = p.bytes() <= room ? unbounded
-                                          : pk_plan_cap(cus, np, band, maxlen, kb_lo, kb_hi, forced, ext, room, cap, p);
+    const double cost = p.bytes() <= room ? unbounded : pk_plan_cap(cus, q, room, cap, p);
     if (cost && (!best_cost || cost < best_cost)) {
       best_cost = cost;
       best = p;
     }
   }
-  return best_cost && best_cost <= 1.6 * free_cost ? best : none;
+  bool beside;
+  const double limit = all_packed ? 1.6 * free_cost : q.us(none.map, 4 * cus, &beside) * (best.beside ? 1.1 : 1);
+  return best_cost && best_cost <= limit ? best : none;
 }
 
 // The DP phase's launches after the bucket sort: the plan, then every family
-// that the reads' kB range allows on its worker stream.  No host read-back and nothing sized by the histogram, so the
+// that the reads' kB range allows on its stream.  No host read-back and nothing sized by the histogram, so the
 // sequence can be captured into a graph.  Per-family timers only with graphs off.
 static int enqueue_dp(crispy_ctx *ctx, const NwFusedArgs &args, const unsigned (&grid)[kNumFamilies],
                       const PkPlan &pk, bool graphs) {
@@ -535,7 +623,8 @@ static int enqueue_dp(crispy_ctx *ctx, const NwFusedArgs &args, const unsigned (
   CRISPY_TRY(fork_workers(ctx));
   for (int f = 0; f < kNumFamilies; ++f) {
     if (!grid[f]) continue;
-    hipStream_t s = ctx->workers[family_worker(f)];
+    const int w = family_stream(f);
+    hipStream_t s = w == kMainStream ? ctx->stream : ctx->workers[w];
     const char *name = f >= kFirstPkFamily ? "nw_band_pk" : f >= kNumRegFamilies ? "nw_band_sliced" : "nw_band_reg";
     hipEvent_t ev = nullptr;
     if (!graphs) timer_begin(ctx, name, &ev, s);
@@ -595,7 +684,8 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
   const int64_t room = ctx->scratch_limit >= 0 ? ctx->scratch_limit
                        : ctx->mem_limit > 0    ? ctx->mem_limit - ctx->dev_bytes + (int64_t)nw.dirs.bytes - later
                                                : kPkScratchBytes;
-  PkPlan pk = pk_plan(ctx->cus, np, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, rs.ext, room);
+  const DpShape shape{np, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, rs.ext};
+  PkPlan pk = pk_plan(ctx->cus, shape, room);
   struct Busy {
     NwState &nw;
     ~Busy() { nw.busy = false; }
@@ -604,15 +694,16 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
     const int rc = ensure(ctx, nw.dirs, (size_t)pk.bytes());
     if (rc == CRISPY_ERR_NOMEM) {  // a device that others fill: the unpacked kernels need no scratch
       ctx->err.clear();
-      pk = pk_plan(ctx->cus, 0, band, rs.maxlen, kb_lo, kb_hi, nw.slice_width, rs.ext, 0);
+      pk = pk_plan(ctx->cus, shape, 0);
     } else if (rc != CRISPY_OK) {
       return rc;
     }
   }
   nw.busy = true;
   for (int f = 0; f < kNumPkFamilies; ++f) {
-    static_assert(kNumWorkers == 2, "the second worker's region follows the first's");
-    pk.args[f].dirs = nw.dirs.as<uint32_t>() + (family_worker(kFirstPkFamily + f) ? pk.region[0] / 4 : 0);
+    // the main stream's region, then the second worker's
+    pk.args[f].dirs = nw.dirs.as<uint32_t>() +
+                      (family_stream(kFirstPkFamily + f) == kMainStream ? 0 : pk.region[kMainStream] / 4);
     pk.args[f].pack_hi = rs.ext ? rs.pack_hi.as<uint32_t>() : nullptr;
   }
   const int ext_top = rs.ext ? pk.map.pk_top : -1;
@@ -649,7 +740,7 @@ static int nw_core(crispy_ctx *ctx, const int2 *d_pairs, int64_t np, int band) {
       (uintptr_t)args.order, (uintptr_t)args.plan, (uintptr_t)args.out, (uintptr_t)nw.hist.p,
       (uintptr_t)nw.cells.p, (uintptr_t)(ctx->timing ? nw.stat.p : nullptr), (uintptr_t)nw.slice_width,
       (uintptr_t)pk.map.pk_top, (uintptr_t)pk.map.pk_cap, (uintptr_t)nw.dirs.p,
-      (uintptr_t)pk.region[0], (uintptr_t)pk.args[0].pack_hi};
+      (uintptr_t)pk.region[kMainStream], (uintptr_t)pk.args[0].pack_hi};
   for (unsigned g : grid) key.push_back(g);
   for (const PkLaunchArgs &k : pk.args) key.push_back((uintptr_t)k.words * 8 + k.block_waves);
   uint64_t kernels = rs.ext ? 1 : 2;
