@@ -34,9 +34,11 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "k-mer pairs/s + banded-NW GCUPS, 1 GPU; served jobs/s with p50/p99 latency"
-VALU_PEAK_TOPS = 78.6    # 256 CU x 64 lanes x 2.4 GHz x 2: the packed NW kernels do two 16-bit operations per lane
+VALU_PEAK_TOPS = 39.3    # 256 CU x 64 lanes x 2.4 GHz: lane instructions/s
 MFMA_FP4_PEAK_TOPS = 10100.0  # MI355X dense FP4 matrix ops/s (10.1 PFLOP/s)
-NW_OPS_PER_CELL = 13     # nominal int ops per in-band DP cell
+# VALU lane instructions per in-band DP cell of the packed NW recurrence (10.3
+# for a lane's two cells); what a step spends beside its cells is not counted
+NW_OPS_PER_CELL = 5.15
 KMER_KERNELS = ("kmer_profile", "kmer_tile", "kmer_cand_pop", "kmer_cand_sort", "kmer_cand", "kmer_sort")
 NW_KERNELS = ("nw_bucket", "nw_band_pk", "nw_band_reg", "nw_band_sliced", "nw_generic", "nw_filter")
 # the NW launches of one step run concurrently on side streams; this event
@@ -469,9 +471,9 @@ def main():
         ach = cells * NW_OPS_PER_CELL / (phase_ms * 1e-3) / 1e12
         traffic, src = measured_traffic(args.workload, "nw_dp_phase")
         roofline = {"kernel": "nw_dp_phase", "bound": "valu", "achieved": ach,
-                    "peak": VALU_PEAK_TOPS, "unit": "Tops/s (16-bit ops, two per lane)",
+                    "peak": VALU_PEAK_TOPS, "unit": "T lane instructions/s",
                     "frac": ach / VALU_PEAK_TOPS,
-                    "work": f"{NW_OPS_PER_CELL} int ops x in-band DP cells ({cells:.4e}/step)",
+                    "work": f"{NW_OPS_PER_CELL} packed lane instructions x in-band DP cells ({cells:.4e}/step)",
                     "phase_ms": phase_ms, "avg_launch_ms": phase_ms,
                     "dp_form": ("kernel launches" if args.no_graphs else
                                 "captured HIP graph: plan kernel + one launch per kernel family"),
