@@ -123,7 +123,7 @@ def measured_traffic(workload, kernel):
     """HBM bytes per launch of `kernel` ("kmer_tile", or "nw_dp_phase": the
     fused family launches of one step) from the committed PMC summary of this
     workload (two rocprofv3 --pmc runs, scaled by a copy kernel of known size),
-    or None when there is none."""
+    or None when there is none.  Counted at the workload's own k."""
     import re
     names = {"kmer_tile": f"kmer_tile_{workload}_counters.md",
              "nw_dp_phase": f"kmer_nw_step_{workload}_traffic.md"}
@@ -469,7 +469,7 @@ def main():
         # One DP phase per step: the fused register / sliced family launches run
         # concurrently on the worker streams; the phase is timed fork to join.
         ach = cells * NW_OPS_PER_CELL / (phase_ms * 1e-3) / 1e12
-        traffic, src = measured_traffic(args.workload, "nw_dp_phase")
+        traffic, src = (None, None) if args.k else measured_traffic(args.workload, "nw_dp_phase")
         roofline = {"kernel": "nw_dp_phase", "bound": "valu", "achieved": ach,
                     "peak": VALU_PEAK_TOPS, "unit": "T lane instructions/s",
                     "frac": ach / VALU_PEAK_TOPS,
@@ -480,7 +480,7 @@ def main():
                     "family_launches_per_step": dp_launches / steps if args.no_graphs else None,
                     "traffic": traffic, "traffic_source": src}
     else:
-        traffic, src = measured_traffic(args.workload, "kmer_tile")
+        traffic, src = (None, None) if args.k else measured_traffic(args.workload, "kmer_tile")
         roofline = {"kernel": "kmer_tile", "bound": "mfma", "achieved": kmer_tile_tops,
                     "peak": MFMA_FP4_PEAK_TOPS, "unit": "TFLOP/s (FP4 MFMA)",
                     "frac": kmer_tile_tops / MFMA_FP4_PEAK_TOPS,
