@@ -23,9 +23,9 @@ constexpr int kMatch = 5;
 constexpr int kNeg = -1000000;
 
 // Largest band half-width kB = (L1+L2)/(2 band) handled by the register
-// resident NW kernel (one template instance per kB).  Full alignments
-// (band <= 1), pairs with non-ACGT bytes and kB > kKbSliceMax run the
-// generic kernel.
+// resident NW kernel (one template instance per kB).  Where the packed kernels
+// (nw_pk.hpp) do not take them, full alignments (band <= 1) and pairs with
+// non-ACGT bytes run the generic kernel, as kB > kKbSliceMax always does.
 constexpr int kKbRegMax = 32;
 // Wider bands up to kKbSliceMax run the lane-sliced kernel (W = 2kB+1 band
 // cells split over up to 64 lanes of 24 cells each).

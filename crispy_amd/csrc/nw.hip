@@ -29,10 +29,13 @@
 //   The register and sliced bodies run as wave tasks of a few fused launches
 //   (one per occupancy family), not one launch per kB bucket.
 //   nw_band_pk (nw_pk.hpp): two positions per register in 16-bit keys, the
-//     directions in a scratch of the context.  Takes every kB whose keys fit
-//     16 bits, full alignments (kB = the longer read) and reads with up to 12
-//     distinct other bytes; what is past that, and a call without room for
-//     the scratch, runs in the kernels above and below.
+//     directions in a scratch of the context.  Can take every kB whose keys
+//     fit 16 bits, full alignments (kB = the longer read) and reads with up to
+//     12 distinct other bytes; takes the kB up to where pk_plan's cost model
+//     has it faster than the kernels above (full alignments and reads with
+//     other bytes, which have only the generic kernel besides: always).  What
+//     is past that, and a call without room for the scratch, runs in the
+//     kernels above and below.
 //   nw_generic_kernel  one lane per pair, the row state in a lane-
 //     interleaved global scratch, raw byte compares.  Any kB, full mode and
 //     reads with other bytes (N, lowercase, ...).

@@ -36,6 +36,14 @@ constexpr int kPkMaxCells = 40;   // 80 state registers: 3 waves per SIMD
 constexpr int kPkMaxLanes = 16;   // lanes per pair
 constexpr int kPkMaxKb = 639;     // 2 kB + 1 positions over kPkMaxLanes x 2 slices of kPkMaxCells
 static_assert(2 * kPkMaxKb + 1 <= 2 * kPkMaxLanes * kPkMaxCells, "the widest band fits the lanes of a pair");
+// The waves are set above what the widest slices' registers leave: the ACGT
+// kernels spill 150, 135, 318 and 241 registers, those with upper code bits 85,
+// 51, 185 and 7, mostly around the steps and not in them.  Measured over six
+// calls: one wave more in every family 0 to 4 % slower (7e3 long reads and reads
+// with N 4 %, 1,000 reads 3 %, 20,000 reads 1 %); one fewer, which spills less,
+// 1.0 to 1.4 % faster with 1e3 to 2.5e5 ACGT reads and 8.5 % with long ones,
+// 0.7 % slower with N.  So the ACGT column may drop by one; the cost model in
+// nw.hip was fitted to the counts here and would have to follow.
 struct PkFamily {
   int lo, hi;     // slice widths
   int waves;      // per SIMD, by registers

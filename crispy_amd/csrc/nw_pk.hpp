@@ -7,14 +7,21 @@
 // ~13.5 instructions per cell (4 selects and 2 compares of them carry the
 // direction, match count and alignment length along every cell).  Here a
 // cell's whole comparison is one integer maximum, and only the end cell's path
-// is ever counted: ~5.3 instructions per cell, the directions' 2 bits written
-// once and the path read back by the wave that wrote it.  Measured (the whole
-// DP phase, before -> now): 0.84 M pairs of 200-300 bp at band 10 3.4 -> 2.2 ms;
-// 3.27 M pairs of 150-550 bp 16.9 -> 9.1 ms; 3000 full alignments of
-// 200-300 bp, which had only the generic kernel, 26.0 -> 0.6 ms; 0.26 M pairs
-// of 300-500 bp, some with N, 17.7 -> 2.3 ms.
-// The second bound at large calls is the directions' traffic: 15 GB out and
-// 20 GB back for 5.0e10 cells, 3.7 TB/s where a copy reaches 4.96.
+// is ever counted: 5.15 instructions per cell in the plain steps, the
+// directions' 2 bits written once and the path read back by the wave that
+// wrote it.  Counted over whole calls, with the boundary and last-column steps,
+// the padding and the trace: 7.3 to 7.7 per in-band cell for 200-900 bp reads
+// at bands 5 and 10, 9.1 for 2000-3200 bp (slices of at most 24 cells), 12 for
+// 1,000 reads and 24 for full alignments, which are boundary steps mostly.
+// Measured (the DP phase, before -> now): 0.84 M pairs of 200-300 bp at band 10
+// 3.4 -> 2.03 ms; 3.27 M pairs of 150-550 bp 16.9 -> 10.2 ms; 0.24 M pairs of
+// 400-900 bp at band 5 12.3 -> 7.0 ms; whole calls with 3000 full alignments of
+// 200-300 bp, which had only the generic kernel, 26.0 -> 0.6 ms, and with reads
+// of 300-500 bp, some with N, 18.2 -> 2.6 ms.
+// The second bound at large calls is the traffic: 15 GB out and 20 GB back for
+// 5.0e10 cells, of which the directions themselves are 12.5 GB each way (the
+// rest is padding, spilled registers and partly used lines), 3.4 TB/s where a
+// copy reaches 4.96.
 //
 // Key of a cell: 4 (M + 11 i - 7 j + off) + p in 16 bits, p = the direction's
 // tie rank (diagonal 3, then 2 and 1: "up" before "left", or "left" before
@@ -94,7 +101,8 @@ __device__ __forceinline__ uint32_t pk_even(uint32_t w) {
 
 // A stream of a read's bases, 16 at a time, from base index q on (any
 // alignment, zeros outside the read).  One word is loaded per 16 bases, two
-// blocks ahead of its use.
+// blocks ahead of its use in the source; the loop that the compiler makes waits
+// for it right after the load, and other waves cover that wait.
 struct PkStream {
   const uint32_t *s;
   int nw, w, sh;        // next word to load, 2 (q mod 16)
@@ -191,7 +199,9 @@ __device__ __forceinline__ void nw_pk_wave(const uint32_t *__restrict__ pack, co
   const int dead_v = W / C, dead_k = W - dead_v * C;
   // (its lanes by execution mask and its cell by masks in scalar registers: a
   // vector mask was spilled, and its reload in every step waited for the
-  // direction stores; choosing the cell by branches moved the row's registers)
+  // direction stores; choosing the cell by branches moved the row's registers.
+  // Of the same kind and still there: the plain steps of the 1-16 and 25-32
+  // families reload the store's 64-bit address from scratch.)
   const bool dead_lane = g == dead_v >> 1;
   const uint32_t dead_half = dead_v & 1 ? 0x0000FFFFu : 0xFFFF0000u;
   uint32_t dead_near[4];  // cells C - 1, - 3, - 5, - 7: where W / (2 G) leaves it mostly
@@ -568,7 +578,8 @@ __device__ __forceinline__ void pk_dispatch(const int c, const NwFusedArgs &a, c
 // Packed kernel for slice widths LO..HI (family F).  The grid is the number
 // of direction slots (about the waves the chip holds), so the scratch is
 // bounded whatever the pair count: a wave keeps its slot and takes the
-// family's tasks one after the other, longest first, from a device counter.
+// family's tasks one after the other, longest first: its slot's number, then
+// what a device counter gives out.
 // Blocks of one wave, or of kPkBlockWaves = 4 independent ones (pk_plan in nw.hip).
 template <int LO, int HI, int WAVES, int F, bool EXT, bool F16>
 __global__ __launch_bounds__(64 * kPkBlockWaves, WAVES) void nw_pk_fused_kernel(const NwFusedArgs a,

@@ -194,10 +194,10 @@ int crispy_nw_csr(crispy_ctx *ctx, int32_t n_rows, int64_t *row_ptr, int32_t *co
 int crispy_nw_set_slice_width(crispy_ctx *ctx, int cells);
 /* Launch form of the context's kernel chains: 1 (the default) = the k-mer
  * profile pass, the k-mer tile pass, the NW DP phase (plan kernel + family
- * kernels) and the NW filter each replay a captured HIP graph, captured on
- * first use and updated (or captured again) when a buffer, a size or a
- * setting changes; 0 = the same kernels launched one by one.  Results do not
- * depend on it.  With graphs on, the context's stream must not itself be
+ * kernels) and the NW filter each replay a captured HIP graph where a run
+ * repeats the one before it (same buffers, sizes and settings; captured on the
+ * second such run, the runs that differ launch their kernels one by one);
+ * 0 = always launched one by one.  Results do not depend on it.  With graphs on, the context's stream must not itself be
  * under capture by the caller.  No counterpart in the reference: a
  * launch-form switch. */
 int crispy_set_graphs(crispy_ctx *ctx, int enable);
